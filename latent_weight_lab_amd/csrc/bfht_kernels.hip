@@ -777,15 +777,13 @@ static hipError_t launch_tile_pass(const BfhtArgs& a, hipStream_t s, int src, in
 // every CU a workgroup, and only with more than one group does a block sum
 // over the groups' rows follow (config 3: 2^20 blocks, 64 blocks in 8 groups,
 // 32 MiB of rows instead of 256 MiB; 2^23, 8 blocks in one group, no rows).
-// Workgroups of the persistent tile passes: one per CU (a workgroup takes all
-// of a CU's LDS), never more than the tiles.
 // The CU count of the current device, cached per device: each slot is written
 // with the same value by whichever thread gets there first (relaxed atomics,
 // so concurrent callers need no lock).
 constexpr int kMaxDevices = 64;
 static std::atomic<int> g_cu_count[kMaxDevices];
 
-static unsigned tile_grid(int64_t ntiles) {
+int64_t device_cus() {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess) dev = -1;
   if (dev >= 0 && dev < kMaxDevices) cus = g_cu_count[dev].load(std::memory_order_relaxed);
@@ -796,8 +794,12 @@ static unsigned tile_grid(int64_t ntiles) {
               : 256;
     if (dev >= 0 && dev < kMaxDevices) g_cu_count[dev].store(cus, std::memory_order_relaxed);
   }
-  return (unsigned)std::min<int64_t>(ntiles, cus);
+  return cus;
 }
+
+// Workgroups of the persistent tile passes: one per CU (a workgroup takes all
+// of a CU's LDS), never more than the tiles.
+static unsigned tile_grid(int64_t ntiles) { return (unsigned)std::min<int64_t>(ntiles, device_cus()); }
 
 template <class T>
 static hipError_t run_tiles(const BfhtArgs& a, hipStream_t s, bool fwd);
@@ -832,7 +834,7 @@ static hipError_t run_tiles(const BfhtArgs& a, hipStream_t s, bool fwd) {
   // the backward's summing last pass: groups of group_blocks blocks, one
   // workgroup per (tile, group), at least as many workgroups as CUs where the
   // blocks allow, no empty group
-  const int64_t cus = tile_grid(INT64_MAX);
+  const int64_t cus = device_cus();
   int64_t ngroups = std::min<int64_t>(std::max<int64_t>((cus + tiles_per_block - 1) / tiles_per_block, 1), a.nblocks);
   const int64_t group_blocks = (a.nblocks + ngroups - 1) / ngroups;
   ngroups = (a.nblocks + group_blocks - 1) / group_blocks;

@@ -47,6 +47,20 @@ struct BfhtArgs {
 
 hipError_t launch_bfht(const BfhtArgs& a, hipStream_t s, bool forward);
 
+// Compute units of the current device (bfht_kernels.hip).
+int64_t device_cus();
+
+// Whether a matrix-core chain launch of `blocks` workgroups (one 2^15 block
+// each) runs its two-per-CU form: one 64 KiB exchange buffer instead of two and
+// at most 128 VGPRs, so two workgroups share a CU and one's loads, stores and
+// barriers overlap the other's stages.  Up to one block per CU the two-buffer
+// form has a barrier less per layer and nothing to overlap with (256 blocks,
+// forward / backward, three layers: 9.1 / 14.3 us either way); beyond, the
+// second round of blocks no longer waits for the first (257 blocks 13.4 -> 10.2
+// and 20.1 -> 16.3 us, 512 blocks 15.3 -> 12.5 and 22.9 -> 19.2 us, 2592 blocks
+// 67.2 -> 53.9 and 107 -> 88 us, block sum included).
+inline bool chains_share_cu(int64_t blocks) { return blocks > device_cus(); }
+
 // Device address of the no-allocation entry's scratch array on the device of
 // stream s (bfht_noalloc.hip), or nullptr with the HIP error in *err.
 void* noalloc_scratch(hipStream_t s, hipError_t* err);

@@ -12,6 +12,57 @@ namespace lwl {
 namespace mfma15 {
 namespace {
 
+// Runs the chain and leaves this lane's eight signed output chunks in v (odd
+// L: from layout F, even L: from S0), times `scale` after their rounding; chunk k
+// holds block positions chunk_pos<L>(x, k) .. + 7.
+template <int L, int kBufs, class SignLayer>
+__device__ __forceinline__ void chain_chunks(const Ctx& x, unsigned char* lds, const u32x4 (&src)[kTiles][2],
+                                             SignLayer sign_layer, u32x4 (&v)[8], float scale = 1.0f) {
+  f32x16 acc[kTiles];
+  uint32_t nw[4];
+  if constexpr (L % 2 == 1) {
+    run_chain<L, true, kBufs>(acc, x, lds, src, sign_layer, nw);
+    direct_chunks(acc, x, reinterpret_cast<const uint32_t*>(lds + kBufs * kXBufBytes) + (L - 1) * kWordsPerLayer, v,
+                  scale);
+  } else {
+    run_chain<L, false, kBufs>(acc, x, lds, src, sign_layer, nw);
+    out_chunks<L>(acc, nw, x, v);
+    if (scale != 1.0f) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = scale_chunk(v[k], scale);
+    }
+  }
+}
+template <int L>
+__device__ __forceinline__ int chunk_pos(const Ctx& x, int k) {
+  return L % 2 == 1 ? direct_chunk_pos(x, k) : out_chunk_pos<L>(x, k);
+}
+
+// Puts the chunks into `lds` in position order (chunk c at stage_slot(c)) and
+// waits for every wave's; returns the staged block.
+template <int L, int kBufs>
+__device__ __forceinline__ const u32x4* stage_chunks(const u32x4 (&v)[8], const Ctx& x, unsigned char* lds) {
+  // two buffers: the one the last layer did not exchange through is free
+  u32x4* stage = reinterpret_cast<u32x4*>(lds + (kBufs == 2 ? (L & 1) * kXBufBytes : 0));
+  if (kBufs == 1) __syncthreads();  // every wave has read the last exchange
+#pragma unroll
+  for (int k = 0; k < 8; ++k) stage[stage_slot(chunk_pos<L>(x, k) >> 3)] = v[k];
+  __syncthreads();
+  return stage;
+}
+
+// The staged block's chunks, consecutive threads on consecutive 16 bytes,
+// write-through; stores past the resource are dropped.
+__device__ __forceinline__ void store_staged(const u32x4* stage, __amdgpu_buffer_rsrc_t out_r) {
+  constexpr int kPer = kChunks / kThreads;
+  u32x4 v[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) v[i] = stage[stage_slot(i * kThreads + (int)threadIdx.x)];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i)
+    __builtin_amdgcn_raw_buffer_store_b128(v[i], out_r, (i * kThreads + (int)threadIdx.x) * 16, 0, kStreamStore);
+}
+
 // ---------------------------------------------------------------- forward
 
 // The 16 bytes that start M bf16 elements before chunk b: the last M elements
@@ -63,43 +114,30 @@ __device__ __forceinline__ void store_range_shifted(const u32x4* stage, __bf16* 
   }
 }
 
-template <int L, bool kWhole>
-__global__ __launch_bounds__(kThreads) void bfht_mfma15_fwd(const __bf16* __restrict__ latent,
-                                                            __bf16* __restrict__ out, int n,
-                                                            int64_t first_block, int64_t start,
-                                                            int64_t stop, uint32_t seed32) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kChainLdsBytes];
-  const int64_t block = first_block + blockIdx.x;
-  const Ctx x = make_ctx(seed32, block);
-  u32x4 src[kTiles][2];
-  load_latent<kWhole>(x, latent, n, src);
-  f32x16 acc[kTiles];
-  uint32_t nw[4];
-  // block-local output range [lo, hi); out element of block position p is (base - start) + p
-  const int64_t base = block * kB;
-  const int lo = kWhole ? 0 : (int)(start - base > 0 ? start - base : 0);
-  const int hi = kWhole ? kB : (int)(stop - base < kB ? stop - base : kB);
-  __bf16* oblk = out + (base - start);
-  const bool full = kWhole || (lo == 0 && hi == kB && (((uintptr_t)oblk & 15) == 0));
-  if constexpr (L % 2 == 1) {
-    // a whole block (uniform): the chain ends in layout F and each lane stores
-    // its chunks directly
-    if (full) {
-      run_chain<L, true>(acc, x, lds, src, [](int i) { return i; }, nw);
-      store_direct(acc, x, reinterpret_cast<const uint32_t*>(lds + kLdsBytes) + (L - 1) * kWordsPerLayer,
-                   rsrc(oblk, (uint32_t)(kB * 2)));
+// Block positions [lo, hi) of the chain's chunks to oblk, every thread of the
+// workgroup (branches uniform).  A whole block on the 16-byte grid (kWhole: the
+// launcher checked that) goes out in whole chunks, from registers where they
+// leave the chain 1 KiB contiguous per wave (odd L); a partial block, or an
+// output off that grid, is staged and stored in aligned 16-byte slots.
+template <int L, int kBufs, bool kWhole = false>
+__device__ __forceinline__ void store_block(const u32x4 (&v)[8], const Ctx& x, unsigned char* lds, __bf16* oblk,
+                                            int lo, int hi) {
+  if (kWhole || (lo == 0 && hi == kB && ((uintptr_t)oblk & 15) == 0)) {
+    const auto out_r = rsrc(oblk, (uint32_t)(kB * 2));
+    if constexpr (L % 2 == 1)
+      store_direct(v, x, out_r);
+    else
+      store_staged(stage_chunks<L, kBufs>(v, x, lds), out_r);
+    return;
+  }
+  if constexpr (!kWhole) {
+    const u32x4* stage = stage_chunks<L, kBufs>(v, x, lds);
+    if ((uintptr_t)oblk & 1) {  // not on the 2-byte grid: element stores
+      uint16_t* o16 = reinterpret_cast<uint16_t*>(oblk);
+      for (int p = lo + (int)threadIdx.x; p < hi; p += kThreads)
+        o16[p] = reinterpret_cast<const uint16_t*>(stage + stage_slot(p >> 3))[p & 7];
       return;
     }
-  }
-  run_chain<L>(acc, x, lds, src, [](int i) { return i; }, nw);
-  // The signed bf16 block goes through the free exchange buffer in position
-  // order, then to memory with consecutive threads on consecutive chunks.
-  u32x4* stage = reinterpret_cast<u32x4*>(lds + (L & 1) * kXBufBytes);
-  stage_output<L>(acc, nw, x, stage);
-  __syncthreads();
-  if (!kWhole && !full && (((uintptr_t)oblk & 1) == 0)) {
-    // part of a block, or an output off the 16-byte grid: 16-byte stores on the
-    // grid, element stores at the range's ends (uniform branch)
     switch (((uintptr_t)oblk >> 1) & 7) {
       case 0: store_range_shifted<0>(stage, oblk, lo, hi); break;
       case 1: store_range_shifted<1>(stage, oblk, lo, hi); break;
@@ -110,28 +148,39 @@ __global__ __launch_bounds__(kThreads) void bfht_mfma15_fwd(const __bf16* __rest
       case 6: store_range_shifted<6>(stage, oblk, lo, hi); break;
       default: store_range_shifted<7>(stage, oblk, lo, hi); break;
     }
-    return;
   }
-  const auto out_r = rsrc(full ? (const void*)oblk : (const void*)out, full ? (uint32_t)(kB * 2) : 0u);
-  uint16_t* oblk16 = reinterpret_cast<uint16_t*>(oblk);
-  constexpr int kPer = kChunks / kThreads;
-  u32x4 v[kPer];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int c = i * kThreads + (int)threadIdx.x;
-    v[i] = stage[stage_slot(c)];
-  }
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int p = (i * kThreads + (int)threadIdx.x) * 8;
-    if (full) {
-      __builtin_amdgcn_raw_buffer_store_b128(v[i], out_r, p * 2, 0, kStreamStore);
-    } else if (p + 8 > lo && p < hi) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (p + e >= lo && p + e < hi) oblk16[p + e] = (uint16_t)(v[i][e >> 1] >> (16 * (e & 1)));
-    }
-  }
+}
+
+// A backward's partial row in whole 16-byte chunks up to its stride (a multiple
+// of 8; the block sum reads only the first n values).
+template <int L, int kBufs>
+__device__ __forceinline__ void store_row(const u32x4 (&v)[8], const Ctx& x, unsigned char* lds, __bf16* row,
+                                          uint32_t row_bytes) {
+  const auto row_r = rsrc(row, row_bytes);
+  if constexpr (L % 2 == 1)
+    store_direct(v, x, row_r);
+  else
+    store_staged(stage_chunks<L, kBufs>(v, x, lds), row_r);
+}
+
+template <int L, bool kWhole, int kBufs>
+__global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_fwd(const __bf16* __restrict__ latent,
+                                                            __bf16* __restrict__ out, int n,
+                                                            int64_t first_block, int64_t start,
+                                                            int64_t stop, uint32_t seed32) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(kBufs)];
+  const int64_t block = first_block + blockIdx.x;
+  const Ctx x = make_ctx(seed32, block);
+  u32x4 src[kTiles][2];
+  load_latent<kWhole>(x, latent, n, src);
+  u32x4 v[8];
+  chain_chunks<L, kBufs>(x, lds, src, [](int i) { return i; }, v);
+  // block-local output range [lo, hi); out element of block position p is (base - start) + p
+  const int64_t base = block * kB;
+  const int lo = kWhole ? 0 : (int)(start - base > 0 ? start - base : 0);
+  const int hi = kWhole ? kB : (int)(stop - base < kB ? stop - base : kB);
+  __bf16* oblk = out + (base - start);
+  store_block<L, kBufs, kWhole>(v, x, lds, oblk, lo, hi);
 }
 
 // ---------------------------------------------------------------- backward
@@ -178,12 +227,12 @@ __device__ __forceinline__ void load_grad_shifted(const Ctx& x, const __bf16* gb
 // formed in float32), half the traffic of float32 rows in both kernels.
 // kWhole: every block's gradient is read whole from a 16-byte aligned place
 // and n % 8 == 0 (the launcher checks), so no partial-chunk paths are needed.
-template <int L, bool kWhole>
-__global__ __launch_bounds__(kThreads) void bfht_mfma15_bwd(const __bf16* __restrict__ grad,
+template <int L, bool kWhole, int kBufs>
+__global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_bwd(const __bf16* __restrict__ grad,
                                                             __bf16* __restrict__ partial, int n,
                                                             int64_t first_block, int64_t start,
                                                             int64_t stop, uint32_t seed32) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kChainLdsBytes];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(kBufs)];
   const int64_t slot = blockIdx.x;
   const int64_t block = first_block + slot;
   const Ctx x = make_ctx(seed32, block);
@@ -223,20 +272,10 @@ __global__ __launch_bounds__(kThreads) void bfht_mfma15_bwd(const __bf16* __rest
         },
         src);
   }
-  f32x16 acc[kTiles];
-  uint32_t nw[4];
-  __bf16* row = partial + slot * mfma15_part_stride(n);
-  if constexpr (L % 2 == 1) {
-    // odd L: the chain ends in layout F and the row goes out from registers,
-    // as the forward's whole blocks do, in whole 16-byte chunks up to the row
-    // stride (n rounded up to 8; the block sum reads only the first n)
-    run_chain<L, true>(acc, x, lds, src, [](int i) { return L - i; }, nw);
-    store_direct(acc, x, reinterpret_cast<const uint32_t*>(lds + kLdsBytes) + (L - 1) * kWordsPerLayer,
-                 rsrc(row, (uint32_t)mfma15_part_stride(n) * 2u));
-    return;
-  }
-  run_chain<L>(acc, x, lds, src, [](int i) { return L - i; }, nw);
-  write_partial_row<L, kWhole, __bf16>(acc, nw, x, lds, row, n, 1.0f);
+  u32x4 v[8];
+  chain_chunks<L, kBufs>(x, lds, src, [](int i) { return L - i; }, v);
+  const int64_t stride = mfma15_part_stride(n);
+  store_row<L, kBufs>(v, x, lds, partial + slot * stride, (uint32_t)stride * 2u);
 }
 
 // ---------------------------------------------------------------- grouped
@@ -244,63 +283,27 @@ __global__ __launch_bounds__(kThreads) void bfht_mfma15_bwd(const __bf16* __rest
 
 // Whole weight of each job (positions [0, size)): the chain of bfht_mfma15_fwd,
 // the bf16 output times the job's weight scale.
-template <int L>
-__global__ __launch_bounds__(kThreads) void bfht_mfma15_fwd_grouped(const GroupTable g) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kChainLdsBytes];
+template <int L, int kBufs>
+__global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_fwd_grouped(const GroupTable g) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(kBufs)];
   const int j = group_job(g, (int)blockIdx.x);
   const GroupJob& jb = g.job[j];
   const int64_t block = (int64_t)blockIdx.x - g.prefix[j];
   const Ctx x = make_ctx(jb.seed32, block);
   u32x4 src[kTiles][2];
   load_latent(x, static_cast<const __bf16*>(jb.src), jb.n, src);
-  f32x16 acc[kTiles];
-  uint32_t nw[4];
+  u32x4 v[8];
+  chain_chunks<L, kBufs>(x, lds, src, [](int i) { return i; }, v, jb.scale);
   const int64_t base = block * kB;
   const int hi = jb.size - base < kB ? (int)(jb.size - base) : kB;
-  __bf16* oblk = static_cast<__bf16*>(jb.dst) + base;
-  const bool full = hi == kB && (((uintptr_t)oblk & 15) == 0);
-  if constexpr (L % 2 == 1) {
-    // a whole block (uniform): layout F, direct stores, as bfht_mfma15_fwd
-    if (full) {
-      run_chain<L, true>(acc, x, lds, src, [](int i) { return i; }, nw);
-      store_direct(acc, x, reinterpret_cast<const uint32_t*>(lds + kLdsBytes) + (L - 1) * kWordsPerLayer,
-                   rsrc(oblk, (uint32_t)(kB * 2)), jb.scale);
-      return;
-    }
-  }
-  run_chain<L>(acc, x, lds, src, [](int i) { return i; }, nw);
-  u32x4* stage = reinterpret_cast<u32x4*>(lds + (L & 1) * kXBufBytes);
-  stage_output<L>(acc, nw, x, stage);
-  __syncthreads();
-  const auto out_r = rsrc(full ? (const void*)oblk : jb.dst, full ? (uint32_t)(kB * 2) : 0u);
-  uint16_t* oblk16 = reinterpret_cast<uint16_t*>(oblk);
-  const float scale = jb.scale;
-  constexpr int kPer = kChunks / kThreads;
-  u32x4 v[kPer];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int c = i * kThreads + (int)threadIdx.x;
-    v[i] = stage[stage_slot(c)];
-    if (scale != 1.0f) v[i] = scale_chunk(v[i], scale);
-  }
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int p = (i * kThreads + (int)threadIdx.x) * 8;
-    if (full) {
-      __builtin_amdgcn_raw_buffer_store_b128(v[i], out_r, p * 2, 0, kStreamStore);
-    } else if (p < hi) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (p + e < hi) oblk16[p + e] = (uint16_t)(v[i][e >> 1] >> (16 * (e & 1)));
-    }
-  }
+  store_block<L, kBufs>(v, x, lds, static_cast<__bf16*>(jb.dst) + base, 0, hi);
 }
 
 // Per-block partial rows of each job's whole-weight gradient (bf16 weight
 // gradient, as bfht_mfma15_bwd), into the job's partial rows.
-template <int L>
-__global__ __launch_bounds__(kThreads) void bfht_mfma15_bwd_grouped(const GroupTable g) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kChainLdsBytes];
+template <int L, int kBufs>
+__global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_bwd_grouped(const GroupTable g) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(kBufs)];
   const int j = group_job(g, (int)blockIdx.x);
   const GroupJob& jb = g.job[j];
   const int64_t slot = (int64_t)blockIdx.x - g.prefix[j];
@@ -340,19 +343,10 @@ __global__ __launch_bounds__(kThreads) void bfht_mfma15_bwd_grouped(const GroupT
         },
         src);
   }
-  f32x16 acc[kTiles];
-  uint32_t nw[4];
-  __bf16* row = static_cast<__bf16*>(jb.part) + slot * (int64_t)jb.stride;
-  if constexpr (L % 2 == 1) {
-    // odd L: the row from layout F in whole 16-byte chunks up to the row stride
-    // (a multiple of 64; the block sum reads only the first n), as bfht_mfma15_bwd
-    run_chain<L, true>(acc, x, lds, src, [](int i) { return L - i; }, nw);
-    store_direct(acc, x, reinterpret_cast<const uint32_t*>(lds + kLdsBytes) + (L - 1) * kWordsPerLayer,
-                 rsrc(row, (uint32_t)jb.stride * 2u));
-    return;
-  }
-  run_chain<L>(acc, x, lds, src, [](int i) { return L - i; }, nw);
-  write_partial_row<L, false, __bf16>(acc, nw, x, lds, row, jb.n, 1.0f);
+  u32x4 v[8];
+  chain_chunks<L, kBufs>(x, lds, src, [](int i) { return L - i; }, v);
+  // the row stride is a multiple of 64
+  store_row<L, kBufs>(v, x, lds, static_cast<__bf16*>(jb.part) + slot * (int64_t)jb.stride, (uint32_t)jb.stride * 2u);
 }
 
 }  // namespace
@@ -369,7 +363,7 @@ bool mfma15_applicable(const BfhtArgs& a, bool fwd) {
 
 namespace {
 
-template <bool kWhole>
+template <bool kWhole, int kBufs>
 hipError_t launch_mfma15_shape(const BfhtArgs& a, hipStream_t s, bool fwd) {
   using namespace mfma15;
   const dim3 grid((unsigned)a.nblocks), block(kThreads);
@@ -378,18 +372,18 @@ hipError_t launch_mfma15_shape(const BfhtArgs& a, hipStream_t s, bool fwd) {
   if (fwd) {
     auto* dst = (__bf16*)a.dst;
     switch (a.layers) {
-      case 1: hipLaunchKernelGGL((bfht_mfma15_fwd<1, kWhole>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
-      case 2: hipLaunchKernelGGL((bfht_mfma15_fwd<2, kWhole>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
-      case 3: hipLaunchKernelGGL((bfht_mfma15_fwd<3, kWhole>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
+      case 1: hipLaunchKernelGGL((bfht_mfma15_fwd<1, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
+      case 2: hipLaunchKernelGGL((bfht_mfma15_fwd<2, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
+      case 3: hipLaunchKernelGGL((bfht_mfma15_fwd<3, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
       default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
   }
   auto* part = (__bf16*)a.work;  // bf16 partial rows (summed in float32, bfht_reduce_blocks)
   switch (a.layers) {
-    case 1: hipLaunchKernelGGL((bfht_mfma15_bwd<1, kWhole>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
-    case 2: hipLaunchKernelGGL((bfht_mfma15_bwd<2, kWhole>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
-    case 3: hipLaunchKernelGGL((bfht_mfma15_bwd<3, kWhole>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
+    case 1: hipLaunchKernelGGL((bfht_mfma15_bwd<1, kWhole, kBufs>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
+    case 2: hipLaunchKernelGGL((bfht_mfma15_bwd<2, kWhole, kBufs>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
+    case 3: hipLaunchKernelGGL((bfht_mfma15_bwd<3, kWhole, kBufs>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -401,11 +395,16 @@ hipError_t launch_mfma15_grouped(const GroupTable& g, int layers, hipStream_t s,
   using namespace mfma15;
   if (g.count <= 0 || g.prefix[g.count] == 0) return hipSuccess;
   const dim3 grid((unsigned)g.prefix[g.count]), block(kThreads);
-#define LWL_GROUPED(L)                                                       \
-  if (fwd)                                                                   \
-    hipLaunchKernelGGL((bfht_mfma15_fwd_grouped<L>), grid, block, 0, s, g); \
-  else                                                                       \
-    hipLaunchKernelGGL((bfht_mfma15_bwd_grouped<L>), grid, block, 0, s, g)
+  const bool paired = chains_share_cu(g.prefix[g.count]);
+#define LWL_GROUPED(L)                                                                      \
+  if (fwd && paired)                                                                        \
+    hipLaunchKernelGGL((bfht_mfma15_fwd_grouped<L, 1>), grid, block, 0, s, g);              \
+  else if (fwd)                                                                             \
+    hipLaunchKernelGGL((bfht_mfma15_fwd_grouped<L, 2>), grid, block, 0, s, g);              \
+  else if (paired)                                                                          \
+    hipLaunchKernelGGL((bfht_mfma15_bwd_grouped<L, 1>), grid, block, 0, s, g);              \
+  else                                                                                      \
+    hipLaunchKernelGGL((bfht_mfma15_bwd_grouped<L, 2>), grid, block, 0, s, g)
   switch (layers) {
     case 1: LWL_GROUPED(1); break;
     case 2: LWL_GROUPED(2); break;
@@ -422,7 +421,9 @@ hipError_t launch_mfma15(const BfhtArgs& a, hipStream_t s, bool fwd) {
   // slice base (out / grad) is 16-byte aligned, so every block's base is too
   const bool whole = a.start == a.first_block * kB && a.stop == (a.first_block + a.nblocks) * kB &&
                      (uintptr_t)a.dst % 16 == 0 && (uintptr_t)a.src % 16 == 0 && a.n % 8 == 0;
-  return whole ? launch_mfma15_shape<true>(a, s, fwd) : launch_mfma15_shape<false>(a, s, fwd);
+  if (chains_share_cu(a.nblocks))
+    return whole ? launch_mfma15_shape<true, 1>(a, s, fwd) : launch_mfma15_shape<false, 1>(a, s, fwd);
+  return whole ? launch_mfma15_shape<true, 2>(a, s, fwd) : launch_mfma15_shape<false, 2>(a, s, fwd);
 }
 
 }  // namespace lwl

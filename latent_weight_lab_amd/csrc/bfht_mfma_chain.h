@@ -71,11 +71,13 @@ constexpr int kXBufBytes = kChunks * 16;
 constexpr int kLdsBytes = 2 * kXBufBytes;
 // Sign-word table after the exchange buffers: the words of sign layers 1..L
 // (1024 per layer, 32 positions each), hashed once per block while the
-// block's source loads are in flight.  A chain kernel's LDS is kChainLdsBytes.
+// block's source loads are in flight.  A chain kernel's LDS is
+// chain_lds_bytes(its exchange buffers).
 constexpr int kMaxChainLayers = 3;
 constexpr int kWordsPerLayer = kB / 32;
 constexpr int kWordTableBytes = kMaxChainLayers * kWordsPerLayer * 4;
-constexpr int kChainLdsBytes = kLdsBytes + kWordTableBytes;
+__host__ __device__ constexpr int chain_lds_bytes(int bufs) { return bufs * kXBufBytes + kWordTableBytes; }
+constexpr int kChainLdsBytes = chain_lds_bytes(2);
 constexpr uint32_t kPairSign = 0x80008000u;
 
 __device__ __forceinline__ uint32_t pk(float lo, float hi) {
@@ -464,7 +466,7 @@ static_assert(unshuffle_bits(0x55555555u) == 0x0000ffffu && unshuffle_bits(0xaaa
                   unshuffle_bits(0x00000006u) == 0x00010002u && unshuffle_bits(0x80000000u) == 0x80000000u,
               "unshuffle_bits");
 
-// Fills the sign-word table (bytes kLdsBytes.. of the chain's LDS): slot j - 1
+// Fills the sign-word table (after the exchange buffers in the chain's LDS): slot j - 1
 // holds the 1024 inverted words of sign layer sign_layer(j), j = 1..L, two per
 // thread, in the form their reader applies: sign layer j < L is read by kernel
 // layer j, whose stage a runs in S1 (j odd: bit permutation swap_idx34) or S0
@@ -521,17 +523,19 @@ __device__ __forceinline__ void read_words(const Ctx& x, const uint32_t* wtab, i
 // in S1 (L odd) or S0 (L even).  Layer i exchanges through buffer i & 1 of
 // `lds`: the previous readers of that buffer (layer i - 2) are past layer
 // i - 1's barrier, and buffer L & 1 needs no barrier before its next writes.
-// `lds` spans kChainLdsBytes; the sign words of layers 1..L are hashed into
+// With kBufs = 1 (workgroups that share a CU) every layer exchanges through the
+// one buffer, after one more barrier.
+// `lds` spans chain_lds_bytes(kBufs); the sign words of layers 1..L are hashed into
 // its table first (their loads' latency covers the hashing) and read after
 // each layer's exchange barrier, which also orders the table's writes.
 // kDirect (odd L): the last layer ends in layout F (see exchange_slot_final)
 // instead of S1, and `fin` is not read (store_direct reads the last words).
-template <int L, bool kDirect = false, class SignLayer>
+template <int L, bool kDirect = false, int kBufs = 2, class SignLayer>
 __device__ __forceinline__ void run_chain(f32x16 (&acc)[kTiles], const Ctx& x, unsigned char* lds,
                                           const u32x4 (&src)[kTiles][2], SignLayer sign_layer,
                                           uint32_t (&fin)[4]) {
   static_assert(!kDirect || L % 2 == 1, "layout F follows an even layer's stages a, b");
-  uint32_t* wtab = reinterpret_cast<uint32_t*>(lds + kLdsBytes);
+  uint32_t* wtab = reinterpret_cast<uint32_t*>(lds + kBufs * kXBufBytes);
   uint32_t nw[L][4];
   layer_words<false>(x, sign_layer(0), nw[0]);
   fill_words<L, kDirect>(x, wtab, sign_layer);
@@ -566,7 +570,8 @@ __device__ __forceinline__ void run_chain(f32x16 (&acc)[kTiles], const Ctx& x, u
       stage_rows<true, false>(acc, hq4, nw[i]);
     }
     stage_rows<false, false>(acc, hq8, nw[i]);
-    u32x2* xbuf = reinterpret_cast<u32x2*>(lds + (i & 1) * kXBufBytes);
+    u32x2* xbuf = reinterpret_cast<u32x2*>(lds + (kBufs == 2 ? (i & 1) * kXBufBytes : 0));
+    if (kBufs == 1 && i > 0) __syncthreads();  // every wave has read layer i - 1's exchange
     if (direct)
       exchange_write_final(acc, xbuf, x);
     else
@@ -769,18 +774,6 @@ __device__ __forceinline__ void out_chunks(const f32x16 (&acc)[kTiles], const ui
 // place as a whole, so reads of consecutive chunks are conflict-free too.
 __device__ __forceinline__ int stage_slot(int c) { return c ^ ((c >> 3) & 3); }
 
-// Stages the chain's result (acc, before the last sign layer, words `nw`) as
-// signed bf16 in block-position order into `stage` (4096 16-byte chunks at
-// stage_slot(c)).  The caller synchronizes before reading.
-template <int L>
-__device__ __forceinline__ void stage_output(const f32x16 (&acc)[kTiles], const uint32_t (&nw)[4], const Ctx& x,
-                                             u32x4* stage) {
-  u32x4 v[8];
-  out_chunks<L>(acc, nw, x, v);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) stage[stage_slot(out_chunk_pos<L>(x, k) >> 3)] = v[k];
-}
-
 // The 8 bf16 of a chunk times `scale`, rounded to bf16 (torch's bf16 * scalar).
 __device__ __forceinline__ u32x4 scale_chunk(u32x4 v, float scale) {
 #pragma unroll
@@ -789,23 +782,22 @@ __device__ __forceinline__ u32x4 scale_chunk(u32x4 v, float scale) {
   return v;
 }
 
-// The forward's whole block from layout F (run_chain<L, true>): the last sign
-// layer and 16-byte write-through stores of whole chunks, 1 KiB contiguous per
-// instruction, straight from registers.  `words` is the table slot the chain
-// filled for it (fill_words<L, true>): a lane's eight words, those of its chunks
-// k = 0..7, are consecutive; the chunk's bit-in-word bits are p0-p2 (in the
+// This lane's eight output chunks from layout F (run_chain<L, true>), signed by
+// the last sign layer: chunk k holds positions direct_chunk_pos(x, k) .. + 7, so
+// chunk k of a wave's lanes is 1 KiB contiguous.  `words` is the table slot the
+// chain filled for it (fill_words<L, true>): a lane's eight words, those of its
+// chunks k = 0..7, are consecutive; the chunk's bit-in-word bits are p0-p2 (in the
 // chunk) + 8 p3 (l5) + 16 p4 (l32 bit 0), so after the shift by 4 (l5 + 2 p4) of
 // the unshuffled word, bit q (bit 16 + q) holds the sign of the chunk's value 2q
 // (2q + 1), the pair of word q, and (w << (15 - q)) & kPairSign is its mask.
 // Each value is multiplied by `scale` (exact when 1) after its rounding to bf16.
-__device__ __forceinline__ void store_direct(const f32x16 (&acc)[kTiles], const Ctx& x, const uint32_t* words,
-                                             __amdgpu_buffer_rsrc_t out_r, float scale = 1.0f) {
+__device__ __forceinline__ void direct_chunks(const f32x16 (&acc)[kTiles], const Ctx& x, const uint32_t* words,
+                                              u32x4 (&v)[8], float scale = 1.0f) {
   const u32x4* wt = reinterpret_cast<const u32x4*>(words) + 2 * ((x.lane32 >> 1) + 16 * x.wave);
   const u32x4 wa = wt[0], wb = wt[1];
   const int sh = 4 * (x.l5 + 2 * (x.lane32 & 1));
   const uint32_t w[8] = {wa[0] >> sh, wa[1] >> sh, wa[2] >> sh, wa[3] >> sh,
                          wb[0] >> sh, wb[1] >> sh, wb[2] >> sh, wb[3] >> sh};
-  u32x4 v[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k)
 #pragma unroll
@@ -827,103 +819,16 @@ __device__ __forceinline__ void store_direct(const f32x16 (&acc)[kTiles], const 
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = scale_chunk(v[k], scale);
   }
-  const int base = 16 * x.l5 + 32 * x.lane32 + 1024 * x.wave;
+}
+__device__ __forceinline__ int direct_chunk_pos(const Ctx& x, int k) {
+  return 8 * x.l5 + 16 * x.lane32 + 512 * x.wave + 4096 * k;
+}
+
+// 16-byte write-through stores of direct_chunks' values, straight from registers.
+__device__ __forceinline__ void store_direct(const u32x4 (&v)[8], const Ctx& x, __amdgpu_buffer_rsrc_t out_r) {
+  const int base = 2 * direct_chunk_pos(x, 0);
 #pragma unroll
   for (int k = 0; k < 8; ++k) __builtin_amdgcn_raw_buffer_store_b128(v[k], out_r, base + 8192 * k, 0, kStreamStore);
-}
-
-// Slot of 4-float chunk c in write_partial_row's staging.  A ds_write_b128
-// serves 8 consecutive lanes per LDS cycle over 32 banks, a ds_read_b128 16
-// lanes over 64 banks: lanes 0-3, 12-15, 20-23, 24-27 together and lanes 4-7,
-// 8-11, 16-19, 28-31 together (the same for 32-63; measured with two active
-// lanes at a time).  The writes hold chunks 8 apart (chunk bits 3-5 vary over
-// 8 lanes), so bits 3-5 are XORed into bits 0-2 as a permutation; bit 4 going
-// to bit 0 also sets the bf16 reads' pairs of chunks 2 (base + lane) + {0, 1}
-// of each cycle's four lane quads apart (with bits 3-5 in place, two of the
-// quads shared the 16-byte bank groups).
-__device__ __forceinline__ int prow_slot(int c) {
-  return c ^ ((c >> 4) & 1) ^ (((c >> 3) & 1) << 1) ^ (((c >> 5) & 1) << 2);
-}
-
-// Backward tail: applies D_0 (inverted words `nw` of the chain's last sign
-// layer, in the chain's output layout) to the adjoint chain's result and
-// writes scale * the float32 row of the first n block positions to prow,
-// staged through the exchange space (128 KiB; 4-float chunk c at prow_slot(c)).
-// kExact: n % 4 == 0 (whole 16-byte stores; stores past n are dropped).
-template <int L, bool kExact, class P = float>
-__device__ __forceinline__ void write_partial_row(const f32x16 (&acc)[kTiles], const uint32_t (&nw)[4],
-                                                  const Ctx& x, unsigned char* lds, P* prow, int n,
-                                                  float scale) {
-  auto flip = [](float v, uint32_t w, int b) {
-    return __uint_as_float(__float_as_uint(v) ^ ((w << (31 - b)) & 0x80000000u));
-  };
-  f32x4* stage = reinterpret_cast<f32x4*>(lds);  // all 128 KiB
-  // bf16 rows of odd L go out in two halves: register r holds position bit 14
-  // = r >> 3, so the first half's stores leave while the second half is staged.
-  constexpr int kPhases = (L % 2 == 1 && sizeof(P) == 2) ? 2 : 1;
-  __syncthreads();  // every wave has read its last exchange
-  const auto p_r = rsrc(prow, (uint32_t)n * (uint32_t)sizeof(P));
-#pragma unroll
-  for (int ph = 0; ph < kPhases; ++ph) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      if (kPhases > 1 && (r >> 3) != ph) continue;
-      f32x4 v;
-      int p;
-      if constexpr (L % 2 == 1) {
-        // S1: chunk = the 4 tiles at register r (p0, p1 = tile bits)
-        p = (((r >> 1) & 1) << 2) + ((r & 1) << 3) + (x.p4 << 4) + (x.lane32 << 5) + ((x.wave >> 1) << 10) +
-            (x.l5 << 12) + ((r >> 2) << 13);
-        const uint32_t w = nw[r >> 2];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] = scale * flip(acc[t][r], w, (p & 31) + t);
-      } else {
-        // S0: chunk = registers r0 .. r0+3 of tile t (p0, p1 = register bits)
-        const int t = r & 3, r0 = (r >> 2) << 2;
-        p = (t << 2) + (((r0 >> 2) & 1) << 4) + (x.lane32 << 5) + (x.l5 << 10) + ((r0 >> 3) << 11) +
-            (x.wave << 12);
-        const uint32_t w = nw[r0 >> 3];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = scale * flip(acc[t][r0 + e], w, (p & 31) + e);
-      }
-      const int c = p >> 2;
-      stage[prow_slot(c)] = v;
-    }
-    __syncthreads();
-    if constexpr (sizeof(P) == 4) {
-#pragma unroll
-      for (int i = 0; i < (kB / 4) / kThreads; ++i) {
-        const int c = i * kThreads + (int)threadIdx.x;
-        const f32x4 v = stage[prow_slot(c)];
-        const int p = c * 4;
-        if (kExact || p + 4 <= n) {
-          __builtin_amdgcn_raw_buffer_store_b128(v, p_r, p * 4, 0, kStreamStore);  // dropped past n
-        } else if (p < n) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (p + e < n) prow[p + e] = v[e];
-        }
-      }
-    } else {  // bf16 row: two staged chunks (8 positions) per 16-byte store
-      constexpr int kPer = (kB / 8) / kPhases;
-#pragma unroll
-      for (int i = 0; i < kPer / kThreads; ++i) {
-        const int c2 = ph * kPer + i * kThreads + (int)threadIdx.x;
-        const f32x4 a = stage[prow_slot(2 * c2)];
-        const f32x4 b = stage[prow_slot(2 * c2 + 1)];
-        const u32x4 v = {pk(a[0], a[1]), pk(a[2], a[3]), pk(b[0], b[1]), pk(b[2], b[3])};
-        const int p = c2 * 8;
-        if (kExact || p + 8 <= n) {
-          __builtin_amdgcn_raw_buffer_store_b128(v, p_r, p * 2, 0, kStreamStore);  // dropped past n
-        } else if (p < n) {
-          uint16_t* row16 = reinterpret_cast<uint16_t*>(prow);
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (p + e < n) row16[p + e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-        }
-      }
-    }
-  }
 }
 
 // Loads the S0 source operands of a block from the latent (n bf16 elements,
