@@ -77,6 +77,10 @@ constexpr int kMaxNT2 = 6;  // two blocks per workgroup: 16-row tiles (register 
 constexpr int kLinearLdsBytes = 160 * 1024;
 static_assert(kLinearLdsBytes >= kChainLdsBytes && kLinearLdsBytes >= kChain2LdsBytes,
               "the generator chains run in the same LDS");
+// Half of it for one-block tiles whose workgroups share a CU (run_chain with one
+// exchange buffer; see chains_share_cu).
+constexpr int kSharedCuLdsBytes = kLinearLdsBytes / 2;
+static_assert(kSharedCuLdsBytes >= chain_lds_bytes(1), "the one-buffer chain runs in half a CU's LDS");
 
 // output rows a tile of kb blocks can touch, incl. the two partial ones
 __host__ __device__ constexpr int64_t linear_rows(int64_t in_features, int kb) {
@@ -134,9 +138,9 @@ constexpr int kStageBytes = 8 * mfma15::kThreads * 16;
 // into entries whose output columns are never stored, so an exact table leaves
 // that much LDS free).
 constexpr int64_t kExactPitchSlack = 16 * 16;
-int linear_pitch(int64_t in_features, int kb) {
+int linear_pitch(int64_t in_features, int kb, int lds_bytes = kLinearLdsBytes) {
   const int64_t padded = 16 * linear_row_tiles(in_features, kb);
-  return (int)(linear_table_bytes(in_features, padded) <= kLinearLdsBytes ? padded : linear_rows(in_features, kb));
+  return (int)(linear_table_bytes(in_features, padded) <= lds_bytes ? padded : linear_rows(in_features, kb));
 }
 bool linear_pitch_fits(int64_t in_features, int kb) {
   const int pitch = linear_pitch(in_features, kb);
@@ -253,7 +257,10 @@ __global__ __launch_bounds__(256) void bfht_linear_tile_x(const unsigned char* _
 // first linear_lds_steps k steps are read from the LDS table, the rest from
 // this workgroup's overflow in `partial`, written in MFMA B-operand order
 // (per k step and row tile, 64 lanes x 16 bytes) and read with the x stream.
-template <int L, int NT, bool kTiled, int KB, bool kEpi, bool kRowTiles = false, int KG = kGroup, int KD = kDepth>
+// kBufs (KB = 1): the chain's exchange buffers; with one, `lds` is
+// kSharedCuLdsBytes and the table's pitch is the one that fits there.
+template <int L, int NT, bool kTiled, int KB, bool kEpi, bool kRowTiles = false, int KG = kGroup, int KD = kDepth,
+          int kBufs = 2>
 __device__ __forceinline__ void linear_item(const __bf16* __restrict__ x, const __bf16* __restrict__ latent,
                                             __bf16* __restrict__ out, float* __restrict__ partial, int tokens,
                                             int in_f, int out_f, int n, uint32_t seed32, float scale,
@@ -261,6 +268,7 @@ __device__ __forceinline__ void linear_item(const __bf16* __restrict__ x, const 
                                             const LinearEpi& ep, unsigned char* lds, int rows_per_tile = 0) {
   static_assert(!kRowTiles || KB == 2 || KB == 3, "row tiles span two or three generated blocks");
   static_assert(KB != 3 || (kRowTiles && kTiled), "three-block tiles are row tiles over the tiled x");
+  static_assert(kBufs == 2 || KB == 1, "only one-block tiles share a CU");
   const int64_t size = (int64_t)in_f * out_f;
   const int64_t tile_len = kRowTiles ? (int64_t)rows_per_tile * in_f : (int64_t)KB * kB;
   const int64_t g0 = tile * tile_len;                             // first flat position
@@ -355,7 +363,7 @@ __device__ __forceinline__ void linear_item(const __bf16* __restrict__ x, const 
       load_latent(c, latent, n, src);
       f32x16 acc[kTiles];
       uint32_t nw[4];
-      run_chain<L>(acc, c, lds, src, [](int i) { return i; }, nw);
+      run_chain<L, false, kBufs>(acc, c, lds, src, [](int i) { return i; }, nw);
       out_chunks<L>(acc, nw, c, v[0]);
     }
     __syncthreads();  // every wave has read its last exchange
@@ -506,7 +514,8 @@ __device__ __forceinline__ void linear_item(const __bf16* __restrict__ x, const 
   // Tiles from `tend` on are masked.
   auto pass = [&](auto g_const, int tg, int tend) {
     constexpr int G = decltype(g_const)::value;
-    constexpr int D = (G == 1 && KB != 3) ? kDepthSingle : KD;
+    // (8 steps where four row tiles share a CU: 12 would spill at 128 VGPRs)
+    constexpr int D = (G == 1 && KB != 3) ? (kBufs == 1 && NT > 3 ? 8 : kDepthSingle) : KD;
     uint32_t xo[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -746,17 +755,26 @@ __global__ __launch_bounds__(256) void bfht_linear_combine(const float* __restri
 // prefix[j] <= i < prefix[j + 1], work item i - prefix[j] = split * nblocks +
 // block, as the single-matrix kernel's non-tiled, one-block-per-workgroup path
 // (kBias: some job has a bias, applied as the single call's epilogue).
-template <int L, int NT, bool kBias>
-__global__ __launch_bounds__(kThreads) void bfht_linear_mfma15_grouped(const LinearGroupTable g) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kLinearLdsBytes];
+//
+// One block is a long dependency chain (latent loads, three layers with a
+// barrier or two each, the scatter, one short contraction on few waves), so with
+// more blocks than CUs two workgroups share each CU (kBufs = 1): half the LDS
+// each, at most 128 VGPRs, one workgroup's waits filled by the other (the 48
+// matrices of a 12-layer GPT-2-small stack, combine included: 134-139 -> 98-100 us
+// at one token, 173 -> 131 at 64, 320 -> 296 at 200; 8 matrices 28.9 -> 25.3).
+template <int L, int NT, bool kBias, int kBufs>
+__global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_linear_mfma15_grouped(const LinearGroupTable g) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kBufs == 1 ? kSharedCuLdsBytes : kLinearLdsBytes];
   const int j = group_job(g, (int)blockIdx.x);
   const LinearGroupJob& jb = g.job[j];
   const int64_t p = (int64_t)blockIdx.x - g.prefix[j];
   const int split = (int)(p / jb.nblocks);
   const int64_t tile = p - (int64_t)split * jb.nblocks;
   const LinearEpi ep{jb.bias, nullptr, nullptr, nullptr, 0.f};
-  linear_item<L, NT, false, 1, kBias>(jb.x, jb.latent, jb.out, g.partial + jb.partial_off, jb.tokens, jb.in_f, jb.out_f,
-                               jb.n, jb.seed32, jb.scale, jb.token_split, jb.nblocks, jb.pitch, split, tile, ep, lds);
+  // sharing a CU, every pass takes one token tile (a four-tile pass holds ~80 registers more)
+  linear_item<L, NT, false, 1, kBias, false, kBufs == 1 ? 1 : kGroup, kDepth, kBufs>(
+      jb.x, jb.latent, jb.out, g.partial + jb.partial_off, jb.tokens, jb.in_f, jb.out_f, jb.n, jb.seed32, jb.scale,
+      jb.token_split, jb.nblocks, jb.pitch, split, tile, ep, lds);
 }
 
 // The straddling-row sums of every job of a grouped launch: workgroup i serves
@@ -841,29 +859,36 @@ hipError_t launch_linear_L(const LinearArgs& a, hipStream_t s) {
   return launch_linear_L<L, true>(a, (const __bf16*)tiled, partial, s);
 }
 
-template <int L, bool kBias>
+template <int L, bool kBias, int kBufs>
 hipError_t launch_grouped_b(const LinearGroupTable& g, int nt, hipStream_t s) {
   const dim3 grid((unsigned)g.prefix[g.count]), block(mfma15::kThreads);
   switch (nt) {
-    case 1: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 1, kBias>), grid, block, 0, s, g); break;
-    case 2: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 2, kBias>), grid, block, 0, s, g); break;
-    case 3: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 3, kBias>), grid, block, 0, s, g); break;
-    case 4: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 4, kBias>), grid, block, 0, s, g); break;
+    case 1: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 1, kBias, kBufs>), grid, block, 0, s, g); break;
+    case 2: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 2, kBias, kBufs>), grid, block, 0, s, g); break;
+    case 3: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 3, kBias, kBufs>), grid, block, 0, s, g); break;
+    case 4: hipLaunchKernelGGL((bfht_linear_mfma15_grouped<L, 4, kBias, kBufs>), grid, block, 0, s, g); break;
     default: return hipErrorInvalidValue;
   }
   return hipSuccess;
 }
 
 template <int L>
-hipError_t launch_grouped_nt(const LinearGroupTable& g, int nt, hipStream_t s) {
+hipError_t launch_grouped_nt(const LinearGroupTable& g, int nt, bool share_cu, hipStream_t s) {
   bool bias = false;
   for (int i = 0; i < g.count; ++i) bias = bias || g.job[i].bias;
-  const hipError_t e0 = bias ? launch_grouped_b<L, true>(g, nt, s) : launch_grouped_b<L, false>(g, nt, s);
+  const hipError_t e0 = bias ? (share_cu ? launch_grouped_b<L, true, 1>(g, nt, s) : launch_grouped_b<L, true, 2>(g, nt, s))
+                             : (share_cu ? launch_grouped_b<L, false, 1>(g, nt, s) : launch_grouped_b<L, false, 2>(g, nt, s));
   if (e0 != hipSuccess) return e0;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || g.cprefix[g.count] == 0) return e;
   hipLaunchKernelGGL(bfht_linear_combine_grouped, dim3((unsigned)g.cprefix[g.count]), dim3(256), 0, s, g);
   return hipGetLastError();
+}
+
+// Whether a one-block tile's table fits half a CU's LDS (its reads never leave
+// the table: rows past the pitch read a row inside it).
+bool table_fits_shared(int64_t in_features) {
+  return linear_table_bytes(in_features, linear_pitch(in_features, 1, kSharedCuLdsBytes)) <= kSharedCuLdsBytes;
 }
 
 // Whether a job's k-major table can be read as `nt` row tiles: the contraction
@@ -883,8 +908,10 @@ hipError_t launch_group_chunk(const LinearArgs* const* jobs, int count, int nt, 
   LinearGroupTable g{};
   g.count = count;
   int64_t total = 0, min_tiles = INT64_MAX;
+  bool share_cu = true;
   for (int i = 0; i < count; ++i) {
     total += jobs[i]->nblocks_w;
+    share_cu = share_cu && table_fits_shared(jobs[i]->in_features);
     const int64_t tt = (jobs[i]->tokens + kTokTile - 1) / kTokTile;
     min_tiles = tt < min_tiles ? tt : min_tiles;
   }
@@ -893,6 +920,7 @@ hipError_t launch_group_chunk(const LinearArgs* const* jobs, int count, int nt, 
   int64_t split = total >= 256 ? 1 : 256 / total;
   if (split > min_tiles) split = min_tiles;
   if (split < 1) split = 1;
+  share_cu = share_cu && chains_share_cu(total * split);
   // partial rows: offsets from the lowest `work` (every job's lies in one
   // 256-byte-aligned workspace)
   g.partial = (float*)jobs[0]->work;
@@ -914,7 +942,7 @@ hipError_t launch_group_chunk(const LinearArgs* const* jobs, int count, int nt, 
     jb.seed32 = a.seed32;
     jb.scale = a.weight_scale;
     jb.nblocks = (int)a.nblocks_w;
-    jb.pitch = linear_pitch(a.in_features, 1);
+    jb.pitch = linear_pitch(a.in_features, 1, share_cu ? kSharedCuLdsBytes : kLinearLdsBytes);
     jb.token_split = (int)split;
     g.prefix[i] = (int)wg;
     g.cprefix[i] = (int)cw;
@@ -924,9 +952,9 @@ hipError_t launch_group_chunk(const LinearArgs* const* jobs, int count, int nt, 
   g.prefix[count] = (int)wg;
   g.cprefix[count] = (int)cw;
   switch (jobs[0]->layers) {
-    case 1: return launch_grouped_nt<1>(g, nt, s);
-    case 2: return launch_grouped_nt<2>(g, nt, s);
-    case 3: return launch_grouped_nt<3>(g, nt, s);
+    case 1: return launch_grouped_nt<1>(g, nt, share_cu, s);
+    case 2: return launch_grouped_nt<2>(g, nt, share_cu, s);
+    case 3: return launch_grouped_nt<3>(g, nt, share_cu, s);
   }
   return hipErrorInvalidValue;
 }
