@@ -866,7 +866,8 @@ static hipError_t run_typed(const BfhtArgs& a, hipStream_t s, bool fwd) {
   if (mfma15_applicable(a, fwd)) {
     hipError_t e = launch_mfma15(a, s, fwd);
     if (e != hipSuccess || fwd) return e;
-    return launch_reduce<T, bf16>((const bf16*)a.work, a.nblocks, mfma15_part_stride(a.n), a.n, (T*)a.dst, s);
+    return launch_reduce<T, bf16>((const bf16*)a.work, mfma15_bwd_rows(a.nblocks), mfma15_part_stride(a.n), a.n,
+                                  (T*)a.dst, s);
   }
   if (a.log_block <= kTileLog)
     return dispatch_block<T>(a.log_block, fwd, a, s, std::make_integer_sequence<int, kTileLog + 1>{});

@@ -54,11 +54,10 @@ int64_t device_cus();
 // each) runs its two-per-CU form: one 64 KiB exchange buffer instead of two and
 // at most 128 VGPRs, so two workgroups share a CU and one's loads, stores and
 // barriers overlap the other's stages.  Up to one block per CU the two-buffer
-// form has a barrier less per layer and nothing to overlap with (256 blocks,
-// forward / backward, three layers: 9.1 / 14.3 us either way); beyond, the
-// second round of blocks no longer waits for the first (257 blocks 13.4 -> 10.2
-// and 20.1 -> 16.3 us, 512 blocks 15.3 -> 12.5 and 22.9 -> 19.2 us, 2592 blocks
-// 67.2 -> 53.9 and 107 -> 88 us, block sum included).
+// form has a barrier less per layer and nothing to overlap with (256 blocks
+// forward, three layers: 9.1 us either way); beyond, the second round of blocks
+// no longer waits for the first (257 blocks 13.4 -> 10.2 us, 512 blocks 15.3 ->
+// 12.5, 2592 blocks 67.2 -> 53.9; grouped flush of 2592 blocks 156 -> 133).
 inline bool chains_share_cu(int64_t blocks) { return blocks > device_cus(); }
 
 // Device address of the no-allocation entry's scratch array on the device of
@@ -72,6 +71,17 @@ bool mfma15_applicable(const BfhtArgs& a, bool fwd);
 // elements (16-byte aligned), inside the float32-row workspace.
 __host__ __device__ inline int64_t mfma15_part_stride(int64_t n) { return (n + 7) / 8 * 8; }
 hipError_t launch_mfma15(const BfhtArgs& a, hipStream_t s, bool forward);
+// Blocks that one workgroup of the matrix-core backward adds up, and the rows it
+// leaves in `work`: one block per row up to one per CU, beyond that the fewest
+// blocks per row that leave at most one row per CU.
+inline int64_t mfma15_bwd_group(int64_t nblocks) {
+  const int64_t cus = device_cus();
+  return nblocks > cus ? (nblocks + cus - 1) / cus : 1;
+}
+inline int64_t mfma15_bwd_rows(int64_t nblocks) {
+  const int64_t g = mfma15_bwd_group(nblocks);
+  return (nblocks + g - 1) / g;
+}
 hipError_t launch_sign_words(uint32_t seed32, int64_t block, int layer, int64_t first_word,
                              int64_t nwords, uint32_t* out, hipStream_t s);
 

@@ -220,33 +220,41 @@ __device__ __forceinline__ void load_grad_shifted(const Ctx& x, const __bf16* gb
       src);
 }
 
-// Per-block partial latent gradient (first n positions) of the
-// adjoint chain D_0 H D_1 ... H D_L applied to grad scattered into the block.
-// The rows are bfloat16 (the gradient's own type; each of the ~2^8 terms of a
-// position's sum carries one bf16 rounding, ~2^-9 relative, and the sum is
-// formed in float32), half the traffic of float32 rows in both kernels.
-// kWhole: every block's gradient is read whole from a 16-byte aligned place
-// and n % 8 == 0 (the launcher checks), so no partial-chunk paths are needed.
-template <int L, bool kWhole, int kBufs>
-__global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_bwd(const __bf16* __restrict__ grad,
-                                                            __bf16* __restrict__ partial, int n,
-                                                            int64_t first_block, int64_t start,
-                                                            int64_t stop, uint32_t seed32) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(kBufs)];
-  const int64_t slot = blockIdx.x;
-  const int64_t block = first_block + slot;
-  const Ctx x = make_ctx(seed32, block);
-  const int64_t base = block * kB;
-  const int lo = kWhole ? 0 : (int)(start - base > 0 ? start - base : 0);
-  const int hi = kWhole ? kB : (int)(stop - base < kB ? stop - base : kB);
-  const __bf16* gblk = grad + (base - start);
-  const bool full = kWhole || (lo == 0 && hi == kB && (((uintptr_t)gblk & 15) == 0));
-  const auto g_r = rsrc(full ? (const void*)gblk : (const void*)grad, full ? (uint32_t)(kB * 2) : 0u);
-  const uint16_t* gblk16 = reinterpret_cast<const uint16_t*>(gblk);
-  u32x4 src[kTiles][2];
-  if (!full && (((uintptr_t)gblk & 1) == 0)) {
-    // part of a block, or a gradient off the 16-byte grid: aligned 16-byte slot loads (uniform branch)
-    const __bf16* gend = grad + (stop - start);
+// Source operands of one block's gradient: positions [lo, hi) of `gblk` (the
+// block's position 0; `gend` is one past the whole gradient), zero elsewhere.
+// kWhole: the whole block, 16-byte aligned.
+__device__ __forceinline__ bool grad_whole(const __bf16* gblk, int lo, int hi) {
+  return lo == 0 && hi == kB && ((uintptr_t)gblk & 15) == 0;
+}
+__device__ __forceinline__ void load_grad_whole(const Ctx& x, const __bf16* gblk, u32x4 (&src)[kTiles][2]) {
+  const auto g_r = rsrc(gblk, (uint32_t)(kB * 2));
+  load_source(x, [&](int p) -> u32x4 { return __builtin_amdgcn_raw_buffer_load_b128(g_r, p * 2, 0, 0); }, src);
+}
+template <bool kWhole>
+__device__ __forceinline__ void load_grad(const Ctx& x, const __bf16* gblk, const __bf16* gend, int lo, int hi,
+                                          u32x4 (&src)[kTiles][2]) {
+  if (kWhole || grad_whole(gblk, lo, hi)) {  // uniform
+    load_grad_whole(x, gblk, src);
+    return;
+  }
+  if constexpr (!kWhole) {
+    if ((uintptr_t)gblk & 1) {  // not on the 2-byte grid: element loads
+      const uint16_t* gblk16 = reinterpret_cast<const uint16_t*>(gblk);
+      load_source(
+          x,
+          [&](int p) -> u32x4 {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (p + 8 > lo && p < hi) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                if (p + e >= lo && p + e < hi) v[e >> 1] |= (uint32_t)gblk16[p + e] << (16 * (e & 1));
+            }
+            return v;
+          },
+          src);
+      return;
+    }
+    // part of a block, or a gradient off the 16-byte grid: aligned 16-byte slot loads
     switch (((uintptr_t)gblk >> 1) & 7) {
       case 0: load_grad_shifted<0>(x, gblk, gend, lo, hi, src); break;
       case 1: load_grad_shifted<1>(x, gblk, gend, lo, hi, src); break;
@@ -257,25 +265,138 @@ __global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_bwd(
       case 6: load_grad_shifted<6>(x, gblk, gend, lo, hi, src); break;
       default: load_grad_shifted<7>(x, gblk, gend, lo, hi, src); break;
     }
+  }
+}
+
+// Per-block partial latent gradient (first n positions) of the
+// adjoint chain D_0 H D_1 ... H D_L applied to grad scattered into the block.
+// The rows are bfloat16 (the gradient's own type; each of the ~2^8 terms of a
+// position's sum carries one bf16 rounding, ~2^-9 relative, and the sum is
+// formed in float32), half the traffic of float32 rows in both kernels.
+// kWhole: every block's gradient is read whole from a 16-byte aligned place
+// and n % 8 == 0 (the launcher checks), so no partial-chunk paths are needed.
+template <int L, bool kWhole>
+__global__ __launch_bounds__(kThreads, 2) void bfht_mfma15_bwd(const __bf16* __restrict__ grad,
+                                                               __bf16* __restrict__ partial, int n,
+                                                               int64_t first_block, int64_t start, int64_t stop,
+                                                               uint32_t seed32) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(2)];
+  const int64_t slot = blockIdx.x;
+  const int64_t block = first_block + slot;
+  const Ctx x = make_ctx(seed32, block);
+  const int64_t base = block * kB;
+  const int lo = kWhole ? 0 : (int)(start - base > 0 ? start - base : 0);
+  const int hi = kWhole ? kB : (int)(stop - base < kB ? stop - base : kB);
+  u32x4 src[kTiles][2];
+  load_grad<kWhole>(x, grad + (base - start), grad + (stop - start), lo, hi, src);
+  u32x4 v[8];
+  chain_chunks<L, 2>(x, lds, src, [](int i) { return L - i; }, v);
+  const int64_t stride = mfma15_part_stride(n);
+  store_row<L, 2>(v, x, lds, partial + slot * stride, (uint32_t)stride * 2u);
+}
+
+// sum += the chain's result signed by its last sign layer, in the chain's end
+// layout: F (odd L, words as direct_chunks reads them) or S0 (even L, words nw).
+template <int L>
+__device__ __forceinline__ void add_signed(f32x16 (&sum)[kTiles], const f32x16 (&acc)[kTiles], const Ctx& x,
+                                           const uint32_t* words, const uint32_t (&nw)[4]) {
+  // both dwords of `pair` shifted left: bit 31 of each is its own word's bit
+  auto shl = [](uint64_t pair, int s) {
+    uint64_t r;
+    asm("v_lshlrev_b64 %0, %1, %2" : "=v"(r) : "s"(s), "v"(pair));
+    return r;
+  };
+  auto add = [&](int t, int r, uint32_t m) {
+    sum[t][r] += __uint_as_float(__float_as_uint(acc[t][r]) ^ (m & 0x80000000u));
+  };
+  if constexpr (L % 2 == 1) {
+    const u32x4* wt = reinterpret_cast<const u32x4*>(words) + 2 * ((x.lane32 >> 1) + 16 * x.wave);
+    const u32x4 wa = wt[0], wb = wt[1];
+    const int sh = 4 * (x.l5 + 2 * (x.lane32 & 1));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint64_t pair = (uint64_t)(wa[k] >> sh) | ((uint64_t)(wb[k] >> sh) << 32);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {  // value j of chunks k and k + 4
+        const uint64_t m = shl(pair, 31 - ((j >> 1) + 16 * (j & 1)));
+        add(j & 3, (j >> 2) | (k << 1), (uint32_t)m);
+        add(j & 3, 8 | (j >> 2) | (k << 1), (uint32_t)(m >> 32));
+      }
+    }
   } else {
-    load_source(
-        x,
-        [&](int p) -> u32x4 {
-          if (full) return __builtin_amdgcn_raw_buffer_load_b128(g_r, p * 2, 0, 0);
-          u32x4 v = {0u, 0u, 0u, 0u};
-          if (p + 8 > lo && p < hi) {
-  #pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (p + e >= lo && p + e < hi) v[e >> 1] |= (uint32_t)gblk16[p + e] << (16 * (e & 1));
-          }
-          return v;
-        },
-        src);
+    const uint64_t pair = (uint64_t)nw[0] | ((uint64_t)nw[1] << 32);  // p11 = 0, 1
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {  // p0-1 = r bits 0-1, p4 = r bit 2, p2-3 = t
+        const uint64_t m = shl(pair, 31 - ((r & 3) + 4 * t + 16 * (r >> 2)));
+        add(t, r, (uint32_t)m);
+        add(t, r + 8, (uint32_t)(m >> 32));
+      }
+  }
+}
+
+// The same over many blocks: workgroup g walks blocks g * group .. of the call in
+// ascending order, adds their chains' results in float32 registers and stores
+// one bfloat16 row, so a call of more blocks than CUs leaves about one row per
+// CU for the block sum instead of one per block, and the next block's gradient
+// loads while the current one transforms.  One workgroup per CU: the chain, the
+// sum (64 registers) and the loads in flight (32) take up to 256 VGPRs.  Three
+// layers, block sum included, against a row per block (two workgroups per CU):
+// 257 blocks 17.8 / 16.3 us, 300 18.1 / 18.4, 600 24.6 / 25.1, 1024 32.2 / 35.2,
+// 2592 67 / 88 (of which the sum of 2592 rows takes 32); a gradient off the
+// 16-byte grid, read without prefetch, 128 / 134 at 2564 blocks.
+template <int L, bool kWhole>
+__global__ __launch_bounds__(kThreads, 2) void bfht_mfma15_bwd_sum(const __bf16* __restrict__ grad,
+                                                                   __bf16* __restrict__ partial, int n,
+                                                                   int64_t first_block, int64_t nblocks,
+                                                                   int64_t group, int64_t start, int64_t stop,
+                                                                   uint32_t seed32) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(2)];
+  const int64_t b0 = (int64_t)blockIdx.x * group, b1 = b0 + group < nblocks ? b0 + group : nblocks;
+  f32x16 sum[kTiles] = {};
+  u32x4 next[kTiles][2];
+  bool loaded = false;  // `next` holds the coming block (a whole, aligned one)
+  Ctx x;
+  for (int64_t b = b0; b < b1; ++b) {
+    x = make_ctx(seed32, first_block + b);
+    const int64_t base = (first_block + b) * kB;
+    const __bf16* gblk = grad + (base - start);
+    if (b > b0) __syncthreads();  // every wave has read the previous block's exchanges and words
+    u32x4 src[kTiles][2];
+    if (loaded) {
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) src[t][c] = next[t][c];
+    } else {
+      const int lo = kWhole ? 0 : (int)(start - base > 0 ? start - base : 0);
+      const int hi = kWhole ? kB : (int)(stop - base < kB ? stop - base : kB);
+      load_grad<kWhole>(x, gblk, grad + (stop - start), lo, hi, src);
+    }
+    // only the last block of a call can be partial after its first
+    loaded = b + 1 < b1 && (kWhole || grad_whole(gblk + kB, 0, (int)(stop - base - kB < kB ? stop - base - kB : kB)));
+    if (loaded) load_grad_whole(x, gblk + kB, next);
+    f32x16 acc[kTiles];
+    uint32_t nw[4];
+    run_chain<L, L % 2 == 1, 2>(acc, x, lds, src, [](int i) { return L - i; }, nw);
+    add_signed<L>(sum, acc, x, reinterpret_cast<const uint32_t*>(lds + 2 * kXBufBytes) + (L - 1) * kWordsPerLayer, nw);
   }
   u32x4 v[8];
-  chain_chunks<L, kBufs>(x, lds, src, [](int i) { return L - i; }, v);
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if constexpr (L % 2 == 1) {  // direct_chunks' order
+        const int r = (q >> 1) | (k << 1);
+        v[k][q] = pk(sum[2 * (q & 1)][r], sum[2 * (q & 1) + 1][r]);
+      } else {  // out_chunks' order
+        const int t = (q >> 1) + 2 * (k & 1), r = 2 * (q & 1) + 4 * ((k >> 1) & 1) + 8 * (k >> 2);
+        v[k][q] = pk(sum[t][r], sum[t][r + 1]);
+      }
+    }
   const int64_t stride = mfma15_part_stride(n);
-  store_row<L, kBufs>(v, x, lds, partial + slot * stride, (uint32_t)stride * 2u);
+  store_row<L, 2>(v, x, lds, partial + (int64_t)blockIdx.x * stride, (uint32_t)stride * 2u);
 }
 
 // ---------------------------------------------------------------- grouped
@@ -310,39 +431,9 @@ __global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_bwd_
   const Ctx x = make_ctx(jb.seed32, slot);
   const int64_t base = slot * kB;
   const int hi = jb.size - base < kB ? (int)(jb.size - base) : kB;
-  const __bf16* gblk = static_cast<const __bf16*>(jb.src) + base;
-  const bool full = hi == kB && (((uintptr_t)gblk & 15) == 0);
-  const auto g_r = rsrc(full ? (const void*)gblk : jb.src, full ? (uint32_t)(kB * 2) : 0u);
-  const uint16_t* gblk16 = reinterpret_cast<const uint16_t*>(gblk);
+  const __bf16* g0 = static_cast<const __bf16*>(jb.src);
   u32x4 src[kTiles][2];
-  if (!full && (((uintptr_t)gblk & 1) == 0)) {
-    // the last, partial block, or a weight gradient off the 16-byte grid (uniform branch)
-    const __bf16* gend = static_cast<const __bf16*>(jb.src) + jb.size;
-    switch (((uintptr_t)gblk >> 1) & 7) {
-      case 0: load_grad_shifted<0>(x, gblk, gend, 0, hi, src); break;
-      case 1: load_grad_shifted<1>(x, gblk, gend, 0, hi, src); break;
-      case 2: load_grad_shifted<2>(x, gblk, gend, 0, hi, src); break;
-      case 3: load_grad_shifted<3>(x, gblk, gend, 0, hi, src); break;
-      case 4: load_grad_shifted<4>(x, gblk, gend, 0, hi, src); break;
-      case 5: load_grad_shifted<5>(x, gblk, gend, 0, hi, src); break;
-      case 6: load_grad_shifted<6>(x, gblk, gend, 0, hi, src); break;
-      default: load_grad_shifted<7>(x, gblk, gend, 0, hi, src); break;
-    }
-  } else {
-    load_source(
-        x,
-        [&](int p) -> u32x4 {
-          if (full) return __builtin_amdgcn_raw_buffer_load_b128(g_r, p * 2, 0, 0);
-          u32x4 v = {0u, 0u, 0u, 0u};
-          if (p < hi) {
-  #pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (p + e < hi) v[e >> 1] |= (uint32_t)gblk16[p + e] << (16 * (e & 1));
-          }
-          return v;
-        },
-        src);
-  }
+  load_grad<false>(x, g0 + base, g0 + jb.size, 0, hi, src);
   u32x4 v[8];
   chain_chunks<L, kBufs>(x, lds, src, [](int i) { return L - i; }, v);
   // the row stride is a multiple of 64
@@ -364,28 +455,43 @@ bool mfma15_applicable(const BfhtArgs& a, bool fwd) {
 namespace {
 
 template <bool kWhole, int kBufs>
-hipError_t launch_mfma15_shape(const BfhtArgs& a, hipStream_t s, bool fwd) {
+hipError_t launch_mfma15_fwd(const BfhtArgs& a, hipStream_t s) {
   using namespace mfma15;
   const dim3 grid((unsigned)a.nblocks), block(kThreads);
   auto* src = (const __bf16*)a.src;
+  auto* dst = (__bf16*)a.dst;
   const int n = (int)a.n;
-  if (fwd) {
-    auto* dst = (__bf16*)a.dst;
-    switch (a.layers) {
-      case 1: hipLaunchKernelGGL((bfht_mfma15_fwd<1, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
-      case 2: hipLaunchKernelGGL((bfht_mfma15_fwd<2, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
-      case 3: hipLaunchKernelGGL((bfht_mfma15_fwd<3, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
-      default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-  }
-  auto* part = (__bf16*)a.work;  // bf16 partial rows (summed in float32, bfht_reduce_blocks)
   switch (a.layers) {
-    case 1: hipLaunchKernelGGL((bfht_mfma15_bwd<1, kWhole, kBufs>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
-    case 2: hipLaunchKernelGGL((bfht_mfma15_bwd<2, kWhole, kBufs>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
-    case 3: hipLaunchKernelGGL((bfht_mfma15_bwd<3, kWhole, kBufs>), grid, block, 0, s, src, part, n, a.first_block, a.start, a.stop, a.seed32); break;
+    case 1: hipLaunchKernelGGL((bfht_mfma15_fwd<1, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
+    case 2: hipLaunchKernelGGL((bfht_mfma15_fwd<2, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
+    case 3: hipLaunchKernelGGL((bfht_mfma15_fwd<3, kWhole, kBufs>), grid, block, 0, s, src, dst, n, a.first_block, a.start, a.stop, a.seed32); break;
     default: return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+template <bool kWhole>
+hipError_t launch_mfma15_bwd(const BfhtArgs& a, hipStream_t s) {
+  using namespace mfma15;
+  const int64_t group = mfma15_bwd_group(a.nblocks);
+  const dim3 grid((unsigned)mfma15_bwd_rows(a.nblocks)), block(kThreads);
+  auto* src = (const __bf16*)a.src;
+  auto* part = (__bf16*)a.work;  // bf16 partial rows (summed in float32, bfht_reduce_blocks)
+  const int n = (int)a.n;
+#define LWL_BWD(L)                                                                                               \
+  if (group > 1)                                                                                                 \
+    hipLaunchKernelGGL((bfht_mfma15_bwd_sum<L, kWhole>), grid, block, 0, s, src, part, n, a.first_block,        \
+                       a.nblocks, group, a.start, a.stop, a.seed32);                                             \
+  else                                                                                                           \
+    hipLaunchKernelGGL((bfht_mfma15_bwd<L, kWhole>), grid, block, 0, s, src, part, n, a.first_block, a.start,   \
+                       a.stop, a.seed32)
+  switch (a.layers) {
+    case 1: LWL_BWD(1); break;
+    case 2: LWL_BWD(2); break;
+    case 3: LWL_BWD(3); break;
+    default: return hipErrorInvalidValue;
+  }
+#undef LWL_BWD
   return hipGetLastError();
 }
 
@@ -421,9 +527,9 @@ hipError_t launch_mfma15(const BfhtArgs& a, hipStream_t s, bool fwd) {
   // slice base (out / grad) is 16-byte aligned, so every block's base is too
   const bool whole = a.start == a.first_block * kB && a.stop == (a.first_block + a.nblocks) * kB &&
                      (uintptr_t)a.dst % 16 == 0 && (uintptr_t)a.src % 16 == 0 && a.n % 8 == 0;
-  if (chains_share_cu(a.nblocks))
-    return whole ? launch_mfma15_shape<true, 1>(a, s, fwd) : launch_mfma15_shape<false, 1>(a, s, fwd);
-  return whole ? launch_mfma15_shape<true, 2>(a, s, fwd) : launch_mfma15_shape<false, 2>(a, s, fwd);
+  if (!fwd) return whole ? launch_mfma15_bwd<true>(a, s) : launch_mfma15_bwd<false>(a, s);
+  if (chains_share_cu(a.nblocks)) return whole ? launch_mfma15_fwd<true, 1>(a, s) : launch_mfma15_fwd<false, 1>(a, s);
+  return whole ? launch_mfma15_fwd<true, 2>(a, s) : launch_mfma15_fwd<false, 2>(a, s);
 }
 
 }  // namespace lwl

@@ -1,6 +1,7 @@
-"""GPU parity of the matrix-core launches whose workgroups share a CU (more generated blocks
-than CUs: one exchange buffer, at most 128 VGPRs): the generator's forward and backward
-against the C oracle, and the grouped fused linear against its single calls.
+"""GPU parity of the matrix-core launches of more generated blocks than CUs: those whose
+workgroups share a CU (one exchange buffer, at most 128 VGPRs: the generator's forward, the
+grouped weight calls, the grouped fused linear) and the backward whose workgroups sum several
+blocks, against the C oracle and against smaller launches or single calls.
 
 A block runs the same arithmetic in both forms, so where a smaller launch (one workgroup per
 CU) covers the same blocks the results are compared bit for bit.
@@ -49,9 +50,11 @@ def test_forward(n, start, cut, layers):
 
 
 @pytest.mark.parametrize("layers", [1, 2, 3])
-@pytest.mark.parametrize("n,start,cut", SHAPES)
-def test_backward(n, start, cut, layers):
-    size = BLOCKS * B
+@pytest.mark.parametrize("blocks,n,start,cut", [(BLOCKS, *s) for s in SHAPES] + [(515, 20001, 0, 9)])
+def test_backward(blocks, n, start, cut, layers):
+    """Groups of 2 (the last one block) and 3 (the last two): whole blocks, blocks off the
+    16-byte grid, and whole blocks read ahead with a partial one at the end."""
+    size = blocks * B
     stop = size - cut
     g = torch.randn(stop - start, generator=torch.Generator().manual_seed(layers + 10)).to(BF16)
     got = ops.backward(g.cuda(), n, BF16, size, layers, SEED, start, stop)
