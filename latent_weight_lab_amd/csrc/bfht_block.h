@@ -202,17 +202,17 @@ struct BlockSeq {
 
 constexpr int kSignTableLayers = 4;  // layers 0..3
 
-template <int LB>
+template <int LB, int kSlots = Geo<LB>::G>  // kSlots: blocks the workgroup transforms together
 struct BlockLds {
   using Gm = Geo<LB>;
   // per block: the padded exchange buffer, then the sign-word table
-  static constexpr int FLOATS = Gm::NG > 1 ? Gm::G * (Gm::PADDED + kSignTableLayers * Gm::TB) : 1;
+  static constexpr int FLOATS = Gm::NG > 1 ? kSlots * (Gm::PADDED + kSignTableLayers * Gm::TB) : 1;
   __device__ static float* data(float* smem, int gi) { return smem + gi * Gm::PADDED; }
   __device__ static uint32_t* table(float* smem, int gi) {
     return reinterpret_cast<uint32_t*>(smem) + table_word(gi);
   }
   // word index of group gi's table from the start of smem
-  __device__ static int table_word(int gi) { return Gm::G * Gm::PADDED + gi * kSignTableLayers * Gm::TB; }
+  __device__ static int table_word(int gi) { return kSlots * Gm::PADDED + gi * kSignTableLayers * Gm::TB; }
 };
 
 // Whether the exchange between groups 1 (bits 0-4) and 2 keeps every value in
@@ -346,7 +346,9 @@ __device__ __forceinline__ void fill_sign_table(uint32_t* tab, uint32_t bkey, in
 // Forward of block slot `slot` (block first_block + slot of one generator) by
 // thread group gi of the workgroup; every thread of the workgroup calls it
 // (barriers inside), threads of an inactive slot (slot >= nblocks) included.
-template <int LB, class T, class Store>
+// kSyncStore: every thread waits before the stores until the exchange buffers
+// are no longer read (for stores that reuse their LDS).
+template <int LB, class T, int kSlots = Geo<LB>::G, bool kSyncStore = false, class Store>
 __device__ __forceinline__ void block_fwd_slot(const T* __restrict__ latent, Store out, int n,
                                                int64_t first_block, int64_t slot, int64_t nblocks, int64_t start,
                                                int64_t stop, uint32_t seed32, int layers, float* smem) {
@@ -359,8 +361,8 @@ __device__ __forceinline__ void block_fwd_slot(const T* __restrict__ latent, Sto
     const int t = threadIdx.x & (Gm::TB - 1);
     const bool active = slot < nblocks;
     const int64_t block = first_block + (active ? slot : 0);
-    float* lds = BlockLds<LB>::data(smem, gi);
-    uint32_t* tab = BlockLds<LB>::table(smem, gi);
+    float* lds = BlockLds<LB, kSlots>::data(smem, gi);
+    uint32_t* tab = BlockLds<LB, kSlots>::table(smem, gi);
     fill_sign_table<LB>(tab, block_key(seed32, block), t, layers);
     // coalesced layout: register r of thread t holds position r * TB + t;
     // positions >= n read 0 (buffer range)
@@ -375,7 +377,7 @@ __device__ __forceinline__ void block_fwd_slot(const T* __restrict__ latent, Sto
     }
     __syncthreads();  // the sign table is complete
     const uint32_t* words = reinterpret_cast<const uint32_t*>(smem);
-    const int tw = BlockLds<LB>::table_word(gi);
+    const int tw = BlockLds<LB, kSlots>::table_word(gi);
     sign_flip<LB>(v, words, tw, t, S::lo(0), S::nb(0));
     for (int layer = 0; layer < layers; ++layer) {
       const bool odd = layer & 1;
@@ -413,12 +415,18 @@ __device__ __forceinline__ void block_fwd_slot(const T* __restrict__ latent, Sto
         }
       }
     };
+    auto drained = [] {
+      if constexpr (kSyncStore) __syncthreads();
+    };
     if (!(layers & 1)) {
+      drained();
       store(S::lo(0), S::nb(0));
     } else if constexpr (S::kLastStores) {
+      drained();
       store(S::lo(S::N - 1), S::nb(S::N - 1));
     } else {
       exchange<LB>(v, lds, t, S::lo(S::N - 1), S::nb(S::N - 1), S::lo(0), S::nb(0), Gm::TB <= 64);
+      drained();
       store(S::lo(0), S::nb(0));
     }
   }

@@ -8,9 +8,12 @@
 //
 // A workgroup owns a tile of consecutive generated blocks (32768 weights for
 // 16-bit I/O, 16384 for float32; whole rows, since in_features divides B) and
-// a range of tokens.  It runs the whole-block VALU generator over the tile,
-// one generator call (G blocks) at a time, and the generator's final stores
-// land, scaled by weight_scale and rounded to the I/O type, in an LDS table of
+// a range of tokens.  It runs the whole-block VALU generator over the tile in
+// one call, 32 weights per thread (1024 threads, 512 for float32: with 8 waves
+// and two calls of 2^14 weights the generator waited out its exchanges on half
+// as many waves), and the generator's final stores land, scaled by weight_scale
+// and rounded to the I/O type, over the exchange buffers once they are read, in a
+// table of
 // 16-byte k-chunks: chunk (kc, r) = W[row0 + r][kc*CH .. kc*CH + CH - 1] at slot
 // kc * pitch + mm_row(kc, r), pitch = rows + 1 (odd, so the generator's stores
 // of consecutive k in one row spread over the LDS banks; the contraction reads
@@ -29,6 +32,12 @@
 // feeds it to four MFMAs (k order permuted alike in A and B).
 // Accumulation in float32; the epilogue (lwl_bfht_linear_forward_ex) is applied
 // in the stores.  The weight never touches memory.
+//
+// Bound by the generator (~14 us per tile of two layers) and, at large batches,
+// by the x stream.  One generator call against two: float16 1024 -> 4096 (latent
+// 16384) 25.5 -> 23.1 us at 16 tokens, 37.2 -> 34.4 at 1000, 79.3 -> 78.0 at 4003;
+// 512 -> 4096 58 -> 49 us and 128 -> 4096 42 -> 35 at 4003; 32 -> 2000 (latent 500)
+// 49.5 -> 26.4 at 1000, where a tile had taken four calls.
 #include "bfht_block.h"
 
 #include <algorithm>
@@ -44,9 +53,10 @@ typedef __bf16 bf16x8m __attribute__((ext_vector_type(8)));
 template <int LB, class T>
 struct MmGeo {
   using Gm = Geo<LB>;
-  static constexpr int EC = Gm::G * Gm::B;                             // weights per generator call
   static constexpr int TILE = sizeof(T) == 2 ? 32768 : 16384;          // weights per workgroup
-  static constexpr int NC = TILE / EC;                                 // generator calls per workgroup
+  // 32 weights per thread, so the whole tile is one generator call
+  static constexpr int WG = TILE / 32;
+  static constexpr int SLOTS = TILE / Gm::B;                           // generated blocks per workgroup
   static constexpr int CH = 16 / (int)sizeof(T);                       // k values per 16-byte chunk
   static constexpr int KSTEP = sizeof(T) == 2 ? 32 : 16;               // k per step (one A load per lane)
   // the table: TILE weights plus one spare chunk per k chunk (pitch = rows + 1;
@@ -54,8 +64,11 @@ struct MmGeo {
   // chunk's reads of row tiles past the tile's rows reach (an item's row tiles
   // run at most 63 rows past the table; their columns are never stored)
   static constexpr int TABLE_BYTES = TILE * (int)sizeof(T) + TILE / (16 * CH) * 16 + 64 * 16;
-  static_assert(TILE % EC == 0, "whole generator calls per workgroup");
-  static_assert(BlockLds<LB>::FLOATS * 4 + TABLE_BYTES <= 160 * 1024, "generator and table fit the LDS");
+  // the table takes over the generator's LDS
+  static constexpr int GEN_BYTES = BlockLds<LB, SLOTS>::FLOATS * 4;
+  static constexpr int LDS_BYTES = TABLE_BYTES > GEN_BYTES ? TABLE_BYTES : GEN_BYTES;
+  static_assert(Gm::LT == LB - 5 && SLOTS * Gm::TB == WG, "32 weights per thread");
+  static_assert(LDS_BYTES <= 160 * 1024, "generator and table fit the LDS");
 };
 
 // Table row of W row r in k chunk kc.  A ds_read_b128 serves 16 lanes per LDS
@@ -110,11 +123,11 @@ __device__ __forceinline__ f32x4m mm16(u32x4m a, u32x4m b, f32x4m c) {
                                                    c, 0, 0, 0);
 }
 
-constexpr int kMmTok = 4;    // token tiles (of 16) per item
 constexpr int kMmDepth = 4;  // x prefetch distance in k steps
 
-template <int LB, class T, int kMmRows>
-__global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small_mm(const T* __restrict__ x,
+// kMmTok: token tiles (of 16) per item.
+template <int LB, class T, int kMmRows, int kMmTok>
+__global__ __launch_bounds__((MmGeo<LB, T>::WG)) void bfht_linear_small_mm(const T* __restrict__ x,
                                                                     const u32x4m* __restrict__ xt,
                                                                     const T* __restrict__ latent,
                                                                     T* __restrict__ out, int tokens, int in_f,
@@ -125,8 +138,7 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small_mm(const T* __r
   using MG = MmGeo<LB, T>;
   constexpr int CH = MG::CH;
   constexpr uint32_t kOff = 0x80000000u;  // buffer offset that reads 0 / drops the store
-  __shared__ float smem[BlockLds<LB>::FLOATS];
-  __shared__ __attribute__((aligned(16))) unsigned char table_raw[MG::TABLE_BYTES];
+  __shared__ __attribute__((aligned(16))) unsigned char table_raw[MG::LDS_BYTES];
   T* tbl = reinterpret_cast<T*>(table_raw);
   const u32x4m* chunks = reinterpret_cast<const u32x4m*>(table_raw);
   const int64_t tile = blockIdx.x;
@@ -136,14 +148,13 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small_mm(const T* __r
   const int rows_wg = MG::TILE >> log_in;  // >= 16 (host check)
   const int pitch = rows_wg + 1;
 
-  // 1. the tile's blocks into the table (inactive slots past the last block
-  //    store nothing: their rows lie past out_features and are never stored)
-  for (int c = 0; c < MG::NC; ++c) {
-    const int64_t slot = (tile * MG::NC + c) * Gm::G + (threadIdx.x >> Gm::LT);
-    block_fwd_slot<LB, T>(latent, TableStore<T>{tbl, base, log_in, pitch, scale}, n, 0, slot, nblocks, 0, size,
-                          seed32, layers, smem);
-    __syncthreads();  // the generator's LDS is reused by the next call; after the last, the table is whole
-  }
+  // 1. the tile's blocks into the table, over the generator's exchange buffers
+  //    once they are read (inactive slots past the last block store nothing:
+  //    their rows lie past out_features and are never stored)
+  const int64_t slot = tile * MG::SLOTS + (threadIdx.x >> Gm::LT);
+  block_fwd_slot<LB, T, MG::SLOTS, true>(latent, TableStore<T>{tbl, base, log_in, pitch, scale}, n, 0, slot, nblocks, 0,
+                                         size, seed32, layers, reinterpret_cast<float*>(table_raw));
+  __syncthreads();  // the table is whole
 
   // 2. items of this split: kMmTok token tiles x kMmRows row tiles, round robin over the waves
   const int row0 = (int)(base >> log_in);
@@ -158,7 +169,7 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small_mm(const T* __r
   const int ngroups_r = (nrt + kMmRows - 1) / kMmRows;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int l16 = lane & 15, kq = lane >> 4;
-  constexpr int kWaves = Gm::WG / 64;
+  constexpr int kWaves = MG::WG / 64;
   const int nsteps = in_f / MG::KSTEP;  // 64 bytes of k per step
   // x: the tiled copy (1 KiB per token tile and step, step-major) or the row-major input
   const bool tiled = xt != nullptr;
@@ -282,9 +293,11 @@ hipError_t launch_mm_lb(const LinearArgs& a, const u32x4m* xt, hipStream_t s) {
   // row tiles per item: the tile's 16-row tiles (rows of one tile, or all of out), at most 4
   const int64_t rows = std::min<int64_t>(MG::TILE >> log_in, a.out_features);
   const int rt = rows > 32 ? 4 : rows > 16 ? 2 : 1;
+  // four token tiles per item, two where four row tiles would leave 16 waves'
+  // 128 VGPRs too few
 #define LWL_MM(RT)                                                                                              \
-  hipLaunchKernelGGL((bfht_linear_small_mm<LB, T, RT>), dim3((unsigned)wtiles, (unsigned)a.token_splits),     \
-                     dim3(Gm::WG), 0, s, (const T*)a.x, xt, (const T*)a.latent, (T*)a.out, (int)a.tokens,      \
+  hipLaunchKernelGGL((bfht_linear_small_mm<LB, T, RT, RT == 4 && sizeof(T) == 2 ? 2 : 4>), dim3((unsigned)wtiles, (unsigned)a.token_splits),     \
+                     dim3(MG::WG), 0, s, (const T*)a.x, xt, (const T*)a.latent, (T*)a.out, (int)a.tokens,      \
                      (int)a.in_features, log_in, (int)a.out_features, (int)a.n, a.nblocks_w, a.seed32, a.layers, \
                      a.weight_scale, a.token_splits, a.epi)
   switch (rt) {
@@ -329,13 +342,19 @@ size_t linear_small_mm_workspace_bytes(const LinearArgs& a) {
 }
 
 int linear_small_mm_token_splits(const LinearArgs& a) {
-  // Each split regenerates its tile (the VALU generator takes ~15 us per 2^14
-  // weights on one CU, as long as the contraction of ~1000 tokens), and one
-  // workgroup fills a CU's LDS: about one workgroup per CU, at least 64 tokens
-  // per split.
+  // Each split regenerates its tile (~14 us per 32768 weights of two layers on
+  // one CU, as long as the contraction of ~1000 tokens): as many workgroups as
+  // run at once and no more (a split past that costs a second round: 1024 ->
+  // 1000 in float32, 4003 tokens, 315 workgroups one per CU 160 us, 504 two per
+  // CU 96), at least 64 tokens per split.  One workgroup per CU; float32 tiles of one
+  // 16-row tile fit two (76 KiB of LDS, 118 VGPRs), whose matrix products then
+  // overlap: 1024 -> 4096 at 4003 tokens 313 -> 299 us, about even at 1000, and
+  // below that the second generation costs more (300 tokens: 50 against 56).
   const int64_t tile = a.dtype == kF32 ? 16384 : 32768;
   const int64_t wtiles = (a.in_features * a.out_features + tile - 1) / tile;
-  int64_t split = (256 + wtiles - 1) / wtiles;
+  const int64_t rows = std::min<int64_t>(tile / a.in_features, a.out_features);
+  const int64_t per_cu = a.dtype == kF32 && rows <= 16 && a.tokens >= 1024 ? 2 : 1;
+  int64_t split = per_cu * 256 / wtiles;
   const int64_t most = (a.tokens + 63) / 64;
   if (split > most) split = most;
   if (split > 65535) split = 65535;
