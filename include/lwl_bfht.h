@@ -94,8 +94,9 @@ int lwl_bfht_check_forward(int dtype, int64_t latent_size, int64_t output_size, 
  * The sum over blocks runs in a fixed order (deterministic, unlike the
  * reference's atomicAdd at .cu:221,493).  grad_out and grad_latent have `dtype`.
  * Arithmetic as lwl_bfht_forward (BF16 at block 2^15: matrix cores, bfloat16
- * operands, float32 accumulation, bfloat16 per-block partial rows summed in
- * float32).
+ * operands, float32 accumulation, bfloat16 partial rows summed in float32: one
+ * per block, or with more blocks than compute units one per group of consecutive
+ * blocks, added up in float32 before the row's rounding).
  */
 size_t lwl_bfht_backward_workspace_size(int64_t latent_size, int64_t output_size, int64_t start,
                                         int64_t stop);
@@ -217,13 +218,17 @@ int lwl_bfht_linear_forward_ex(const void* input, const void* latent, int dtype,
  * its own lwl_bfht_linear_forward call bit for bit.  At decode batch sizes a
  * GPT-2 matrix has 18..72 generated blocks, so one matrix per launch leaves
  * most of the chip idle; jobs the bf16 matrix-core kernel takes with fewer
- * than 256 tokens run together, one launch per layer count for up to 48 jobs;
- * other jobs run as their single calls, so jobs do not run in job order.  All
+ * than 256 tokens run together, one launch per layer count for up to 48 jobs,
+ * and so do jobs of the reference's domain at decode batches (fewer than 16
+ * tokens, or shapes its matrix-core variant does not take with one token range;
+ * in_features <= 1024, at one token <= 4096), one launch per block size for up
+ * to 40 jobs; other jobs run as their single calls, so jobs do not run in job order.  All
  * jobs share `dtype`; outputs must not overlap, and no job's output may overlap
  * another job's input, latent, base or bias (the check rejects both); inputs
  * and latents may be shared.  A job's `epilogue` (NULL:
  * none) is that of lwl_bfht_linear_forward_ex; jobs whose epilogue has only a
- * bias still run grouped, jobs with a base or a row-sum term as single calls.
+ * bias still run grouped, jobs with a row-sum term, or a base outside the
+ * reference's domain, as single calls.
  * Workspace (query with the same jobs): the grouped jobs' own workspaces side
  * by side, plus the largest workspace of the jobs that run as single calls
  * (those run one after another on the stream and share it).

@@ -534,9 +534,14 @@ int lwl_bfht_check_linear_jobs(int dtype, const lwl_bfht_linear_job* jobs, int64
 // reads them all), then one region that the jobs running as single launches
 // reuse one after another (the largest of their workspaces).
 // Grouped: the matrix-core kernel's jobs below its tiled-x batch whose epilogue
-// is at most a bias (the grouped table carries one bias pointer per job).
+// is at most a bias (the grouped table carries one bias pointer per job), and
+// the reference domain's jobs at decode batches, which need no workspace
+// (epilogue at most bias and base).
 bool job_grouped(const lwl::LinearArgs& a) {
   return a.tokens > 0 && linear_uses_mfma(a) && lwl::linear_groupable(a) && !a.epi.base && !a.epi.coef;
+}
+bool job_grouped_small(const lwl::LinearArgs& a) {
+  return a.tokens > 0 && !linear_uses_mfma(a) && lwl::linear_small_groupable(a) && !a.epi.coef;
 }
 
 size_t grouped_ws(const std::vector<lwl::LinearArgs>& v) {
@@ -564,22 +569,27 @@ int lwl_bfht_linear_forward_grouped(int dtype, const lwl_bfht_linear_job* jobs, 
   if (rc) return rc;
   // grouped jobs: their own partial-row slices (256-byte multiples, in job
   // order); the others: one shared region after them, used in turn on the stream
-  std::vector<lwl::LinearArgs> grouped;
+  std::vector<lwl::LinearArgs> grouped, small;
   size_t off = 0;
-  for (auto& a : v)
+  for (auto& a : v) {
     if (job_grouped(a)) {
       a.work = (unsigned char*)workspace + off;
       off += linear_ws(a);
       grouped.push_back(a);
+    } else if (job_grouped_small(a)) {
+      small.push_back(a);
     }
+  }
   for (auto& a : v) {
-    if (a.tokens == 0 || job_grouped(a)) continue;
+    if (a.tokens == 0 || job_grouped(a) || job_grouped_small(a)) continue;
     a.work = linear_ex_ws(a) ? (unsigned char*)workspace + off : nullptr;
     const hipError_t e = launch_linear_ex(a, (hipStream_t)stream);
     if (e != hipSuccess) return hip_status(e, "lwl_bfht_linear_forward_grouped");
   }
-  return hip_status(lwl::launch_linear_grouped(grouped.data(), (int64_t)grouped.size(), (hipStream_t)stream),
-                    "lwl_bfht_linear_forward_grouped");
+  hipError_t e = lwl::launch_linear_small_grouped(small.data(), (int64_t)small.size(), (hipStream_t)stream);
+  if (e == hipSuccess)
+    e = lwl::launch_linear_grouped(grouped.data(), (int64_t)grouped.size(), (hipStream_t)stream);
+  return hip_status(e, "lwl_bfht_linear_forward_grouped");
 }
 
 int lwl_bfht_check_linear_backward_latent(int dtype, int64_t tokens, int64_t in_features,

@@ -178,6 +178,26 @@ constexpr int kLinearSmallMaxLog = 14;
 bool linear_small_applicable(int dtype, int log_block, int64_t in_features);
 int linear_small_token_splits(const LinearArgs& a);  // needs tokens, log_block, nblocks_w
 hipError_t launch_linear_small(const LinearArgs& a, hipStream_t s);
+// Several calls in few launches (decode): one launch per element type and block
+// size, each output as its single call computes it; the epilogue at most a bias
+// and a base.
+constexpr int kSmallGroupMax = 40;  // the table stays below the 4 KiB of kernel arguments
+struct SmallGroupJob {
+  const void *x, *latent;
+  void* out;
+  const void *bias, *base;  // or nullptr
+  int32_t tokens, log_in, out_f, n, nblocks, layers;
+  uint32_t seed32;
+  float scale;
+};
+struct SmallGroupTable {  // passed by value; prefix counts workgroups
+  int32_t count;
+  int32_t prefix[kSmallGroupMax + 1];
+  SmallGroupJob job[kSmallGroupMax];
+};
+static_assert(sizeof(SmallGroupTable) <= 4000, "grouped linear table fits the kernel arguments");
+bool linear_small_groupable(const LinearArgs& a);  // needs token_splits; the caller checks the epilogue
+hipError_t launch_linear_small_grouped(const LinearArgs* jobs, int64_t count, hipStream_t s);
 // The same domain at batches of kLinearMmMinTokens and more, contracted on the
 // matrix cores (bfht_linear_small_mm.hip): blocks of 2^5 .. 2^14, in_features a
 // multiple of 32 (16-bit I/O) or 16 (float32) with at least 16 rows per

@@ -10,13 +10,16 @@
 // the whole-block VALU generator: one block of 2^14 per 512-thread workgroup,
 // or 256 / (B/32) smaller blocks per 256-thread workgroup) and a range of
 // tokens.  It generates its blocks in float32 straight into an LDS weight tile
-// (the generator's final stores land in LDS instead of memory, already scaled
+// (the generator's final stores land in LDS instead of memory, over its own
+// exchange buffers once every thread has read them, already scaled
 // by weight_scale, as the reference scales its shared-memory values), then
 // contracts the tile with its tokens: a team of min(in, 64) lanes computes four
 // tokens of one output row, lanes striding over k, and sums its lanes with
 // butterfly shuffles.  All arithmetic is float32; x and out keep the I/O type.
 // The weight never touches memory.
 #include "bfht_block.h"
+
+#include <vector>
 
 namespace lwl {
 namespace {
@@ -46,25 +49,30 @@ struct LdsWeightStore {
 constexpr int kQuad = 4;  // tokens per team pass
 constexpr int kSpan = 8;  // k iterations of a lane whose x loads are in flight together
 
-template <int LB>
+// LDS of a workgroup: the generator's exchange buffers and sign tables, then
+// (over them, once they are read) the weight tile and the staged x of one token
+// quad.  4096 staged values keep a 2^14 block at 80 KiB, so that two workgroups
+// share a CU (grouped launches); kWide holds as many as the generator's LDS.
+template <int LB, bool kWide>
 struct SmallLinearGeo {
   using Gm = Geo<LB>;
   static constexpr int kTileElems = Gm::G * Gm::B;  // weights generated per workgroup
-  static constexpr int kLdsFloats = BlockLds<LB>::FLOATS + kTileElems;
+  static constexpr int kStage = kWide ? BlockLds<LB>::FLOATS : 4096;
+  static constexpr int kNeed = kTileElems + kStage;
+  static constexpr int kLdsFloats = kNeed > BlockLds<LB>::FLOATS ? kNeed : BlockLds<LB>::FLOATS;
+  static_assert(kLdsFloats * 4 <= 160 * 1024 && (kWide || LB > 14 || kLdsFloats * 8 <= 160 * 1024), "LDS of one CU");
 };
+// staged values of a token quad: one token's when the call has only one
+__host__ __device__ constexpr int64_t small_stage(int64_t tokens, int64_t in_f) { return (tokens == 1 ? 1 : kQuad) * in_f; }
 
-template <int LB, class T>
-__global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small(const T* __restrict__ x,
-                                                                 const T* __restrict__ latent, T* __restrict__ out,
-                                                                 int tokens, int in_f, int log_in, int out_f, int n,
-                                                                 int64_t nblocks, uint32_t seed32, int layers,
-                                                                 float scale, int token_split, LinearEpi ep) {
+template <int LB, class T, bool kWide>
+__device__ __forceinline__ void small_item(const T* __restrict__ x, const T* __restrict__ latent, T* __restrict__ out,
+                                           int tokens, int in_f, int log_in, int out_f, int n, int64_t nblocks,
+                                           uint32_t seed32, int layers, float scale, int token_split, int64_t tile,
+                                           int split, const LinearEpi& ep, float* smem) {
   using Gm = Geo<LB>;
-  using SG = SmallLinearGeo<LB>;
-  __shared__ float smem[SG::kLdsFloats];
-  float* wt = smem + BlockLds<LB>::FLOATS;  // the weight tile, row-major [rows][in]
-  const int64_t tile = blockIdx.x;
-  const int split = blockIdx.y;
+  using SG = SmallLinearGeo<LB, kWide>;
+  float* wt = smem;  // the weight tile, row-major [rows][in]
   const int64_t size = (int64_t)in_f * out_f;
   const int64_t base = tile * SG::kTileElems;
 
@@ -74,8 +82,8 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small(const T* __rest
   const int q0 = split * per_split;
   const int q1 = q0 + per_split < quads ? q0 + per_split : quads;
   const auto x_r = tile_rsrc(x, (uint64_t)tokens * in_f * sizeof(T));
-  const int nstage = kQuad * in_f;
-  const bool staged = nstage <= BlockLds<LB>::FLOATS;
+  const int nstage = (int)small_stage(tokens, in_f);
+  const bool staged = nstage <= SG::kStage;
   // thread's share i0 + e * WG (e < kSpan) of quad q's staged x (tokens past the batch read 0)
   auto stage_load = [&](int q, int i0, float (&v)[kSpan]) {
 #pragma unroll
@@ -94,8 +102,8 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small(const T* __rest
   // 1. the tile's G blocks (inactive slots past the last block store nothing;
   //    their rows lie past out_features and are never read)
   const int64_t slot = tile * Gm::G + (threadIdx.x >> Gm::LT);
-  block_fwd_slot<LB, T>(latent, LdsWeightStore{wt, base, scale}, n, 0, slot, nblocks, 0, size, seed32, layers,
-                        smem);
+  block_fwd_slot<LB, T, Gm::G, true>(latent, LdsWeightStore{wt, base, scale}, n, 0, slot, nblocks, 0, size, seed32,
+                                     layers, smem);
   __syncthreads();
 
   // 2. rows row0 .. row0 + rows - 1 against this split's token quads
@@ -215,12 +223,11 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small(const T* __rest
   using Two = std::integral_constant<int, 2>;
   using Quad = std::integral_constant<int, kQuad>;
   if (staged) {
-    // Each quad's x rows are staged once in the generator's LDS (its exchange
-    // buffers and sign tables, free after the barrier above) and every team
+    // Each quad's x rows are staged once behind the weight tile and every team
     // reads them there: read from memory, all the workgroup's passes (and all
     // the workgroups of an XCD, at decode batches) ask its L2 for the same
     // few lines.  Tokens past the batch stage as 0.
-    float* xs = smem;
+    float* xs = smem + SG::kTileElems;
     for (int q = q0; q < q1; ++q) {
       if (q > q0) __syncthreads();  // every team has read the previous quad
       for (int i0 = (int)threadIdx.x; i0 < nstage; i0 += kSpan * Gm::WG) {
@@ -259,6 +266,35 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small(const T* __rest
   }
 }
 
+template <int LB, class T, bool kWide>
+__global__ __launch_bounds__(Geo<LB>::WG) void bfht_linear_small(const T* __restrict__ x,
+                                                                 const T* __restrict__ latent, T* __restrict__ out,
+                                                                 int tokens, int in_f, int log_in, int out_f, int n,
+                                                                 int64_t nblocks, uint32_t seed32, int layers,
+                                                                 float scale, int token_split, LinearEpi ep) {
+  __shared__ float smem[SmallLinearGeo<LB, kWide>::kLdsFloats];
+  small_item<LB, T, kWide>(x, latent, out, tokens, in_f, log_in, out_f, n, nblocks, seed32, layers, scale, token_split,
+                           blockIdx.x, (int)blockIdx.y, ep, smem);
+}
+
+// Several matrices in one launch (decode): workgroup i serves job j with
+// prefix[j] <= i < prefix[j + 1], tile i - prefix[j] of it, all of its tokens.
+// One matrix is one workgroup per CU, most of whose time is the generator's
+// exchanges and barriers; together two workgroups share each CU and no launch
+// waits for the last one's slowest workgroup (16 float32 matrices 1024 -> 4096,
+// blocks of 2^14, two layers: 181 -> 113 us at one token, 205 -> 122 at 4, 351 ->
+// 204 at 12; 24 matrices of 64 x 256 weights, one workgroup each: 451 -> 27).
+template <int LB, class T>
+__global__ __launch_bounds__(Geo<LB>::WG, 4) void bfht_linear_small_grouped(const SmallGroupTable g) {
+  __shared__ float smem[SmallLinearGeo<LB, false>::kLdsFloats];
+  const int j = group_job(g, (int)blockIdx.x);
+  const SmallGroupJob& jb = g.job[j];
+  const LinearEpi ep{jb.bias, jb.base, nullptr, nullptr, 0.f};
+  small_item<LB, T, false>((const T*)jb.x, (const T*)jb.latent, (T*)jb.out, jb.tokens, 1 << jb.log_in, jb.log_in,
+                           jb.out_f, jb.n, jb.nblocks, jb.seed32, jb.layers, jb.scale, 1,
+                           (int64_t)blockIdx.x - g.prefix[j], 0, ep, smem);
+}
+
 // Float32 sums of the rows of x (the fused linear's row-sum term): one wave per
 // row, lanes striding over k with eight loads in flight, then a fixed butterfly.
 template <class T>
@@ -279,16 +315,60 @@ __global__ __launch_bounds__(256) void bfht_row_sums(const T* __restrict__ x, in
   if (lane == 0) xsum[t] = v;
 }
 
+int log2_of(int64_t v) {
+  int l = 0;
+  while (((int64_t)1 << l) < v) ++l;
+  return l;
+}
+
 template <int LB, class T>
 hipError_t launch_small_lb(const LinearArgs& a, hipStream_t s) {
   using Gm = Geo<LB>;
   const int64_t wtiles = (a.nblocks_w + Gm::G - 1) / Gm::G;
-  int log_in = 0;
-  while (((int64_t)1 << log_in) < a.in_features) ++log_in;
-  hipLaunchKernelGGL((bfht_linear_small<LB, T>), dim3((unsigned)wtiles, (unsigned)a.token_splits), dim3(Gm::WG), 0,
-                     s, (const T*)a.x, (const T*)a.latent, (T*)a.out, (int)a.tokens, (int)a.in_features, log_in,
-                     (int)a.out_features, (int)a.n, a.nblocks_w, a.seed32, a.layers, a.weight_scale,
-                     a.token_splits, a.epi);
+  const int log_in = log2_of(a.in_features);
+  // x of a quad that needs more than the narrow form's staging but fits the wide one's
+  const int64_t nstage = small_stage(a.tokens, a.in_features);
+  const bool wide = LB > 10 && nstage > SmallLinearGeo<LB, false>::kStage && nstage <= SmallLinearGeo<LB, true>::kStage;
+#define LWL_SMALL(W)                                                                                                \
+  hipLaunchKernelGGL((bfht_linear_small<LB, T, W>), dim3((unsigned)wtiles, (unsigned)a.token_splits), dim3(Gm::WG), \
+                     0, s, (const T*)a.x, (const T*)a.latent, (T*)a.out, (int)a.tokens, (int)a.in_features, log_in, \
+                     (int)a.out_features, (int)a.n, a.nblocks_w, a.seed32, a.layers, a.weight_scale,                \
+                     a.token_splits, a.epi)
+  if (wide)
+    LWL_SMALL((LB > 10));
+  else
+    LWL_SMALL(false);
+#undef LWL_SMALL
+  return hipGetLastError();
+}
+
+template <int LB, class T>
+hipError_t launch_small_grouped_lb(const LinearArgs* const* jobs, int count, hipStream_t s) {
+  using Gm = Geo<LB>;
+  SmallGroupTable g{};
+  g.count = count;
+  int64_t wg = 0;
+  for (int i = 0; i < count; ++i) {
+    const LinearArgs& a = *jobs[i];
+    SmallGroupJob& jb = g.job[i];
+    jb.x = a.x;
+    jb.latent = a.latent;
+    jb.out = a.out;
+    jb.bias = a.epi.bias;
+    jb.base = a.epi.base;
+    jb.tokens = (int)a.tokens;
+    jb.log_in = log2_of(a.in_features);
+    jb.out_f = (int)a.out_features;
+    jb.n = (int)a.n;
+    jb.nblocks = (int)a.nblocks_w;
+    jb.layers = a.layers;
+    jb.seed32 = a.seed32;
+    jb.scale = a.weight_scale;
+    g.prefix[i] = (int)wg;
+    wg += (a.nblocks_w + Gm::G - 1) / Gm::G;
+  }
+  g.prefix[count] = (int)wg;
+  hipLaunchKernelGGL((bfht_linear_small_grouped<LB, T>), dim3((unsigned)wg), dim3(Gm::WG), 0, s, g);
   return hipGetLastError();
 }
 
@@ -297,6 +377,14 @@ hipError_t dispatch_small(const LinearArgs& a, hipStream_t s, std::integer_seque
   using Fn = hipError_t (*)(const LinearArgs&, hipStream_t);
   static const Fn table[] = {&launch_small_lb<LBs, T>...};
   return table[a.log_block](a, s);
+}
+
+template <class T, int... LBs>
+hipError_t dispatch_small_grouped(int log_block, const LinearArgs* const* jobs, int count, hipStream_t s,
+                                  std::integer_sequence<int, LBs...>) {
+  using Fn = hipError_t (*)(const LinearArgs* const*, int, hipStream_t);
+  static const Fn table[] = {&launch_small_grouped_lb<LBs, T>...};
+  return table[log_block](jobs, count, s);
 }
 
 }  // namespace
@@ -318,6 +406,40 @@ int linear_small_token_splits(const LinearArgs& a) {
   if (split > cap) split = cap;
   if (split > 65535) split = 65535;
   return (int)(split < 1 ? 1 : split);
+}
+
+bool linear_small_groupable(const LinearArgs& a) {
+  // calls of one token range whose staged quad fits the narrow form; their block
+  // count and tile count stay far below 2^31 (tokens * out and in * out do)
+  return linear_small_applicable(a.dtype, a.log_block, a.in_features) && !linear_small_mm_applicable(a) &&
+         a.token_splits == 1 && a.nblocks_w < ((int64_t)1 << 24) &&
+         small_stage(a.tokens, a.in_features) <= SmallLinearGeo<kLinearSmallMaxLog, false>::kStage;
+}
+
+hipError_t launch_linear_small_grouped(const LinearArgs* jobs, int64_t count, hipStream_t s) {
+  // one launch per (type, block size) of up to kSmallGroupMax jobs, buckets in
+  // order of their first job
+  using Seq = std::make_integer_sequence<int, kLinearSmallMaxLog + 1>;
+  std::vector<bool> done((size_t)count, false);
+  std::vector<const LinearArgs*> bucket;
+  for (int64_t i = 0; i < count; ++i) {
+    if (done[(size_t)i]) continue;
+    bucket.clear();
+    for (int64_t k = i; k < count && (int)bucket.size() < kSmallGroupMax; ++k)
+      if (!done[(size_t)k] && jobs[k].dtype == jobs[i].dtype && jobs[k].log_block == jobs[i].log_block) {
+        done[(size_t)k] = true;
+        bucket.push_back(&jobs[k]);
+      }
+    hipError_t e = hipErrorInvalidValue;
+    const int lb = jobs[i].log_block, m = (int)bucket.size();
+    switch (jobs[i].dtype) {
+      case kF32: e = dispatch_small_grouped<float>(lb, bucket.data(), m, s, Seq{}); break;
+      case kF16: e = dispatch_small_grouped<f16>(lb, bucket.data(), m, s, Seq{}); break;
+      case kBF16: e = dispatch_small_grouped<bf16>(lb, bucket.data(), m, s, Seq{}); break;
+    }
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_row_sums(const LinearArgs& a, float* xsum, hipStream_t s) {
