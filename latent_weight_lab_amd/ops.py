@@ -7,6 +7,7 @@ tensors' device.  Nothing here computes on the CPU.
 from __future__ import annotations
 
 import ctypes
+import struct
 
 import torch
 
@@ -245,22 +246,26 @@ def linear_backward_latent(grad2d: torch.Tensor, x2d: torch.Tensor, latent: torc
     return grad_latent
 
 
-def _weight_job(latent: torch.Tensor, size: int, layers: int, seed: int, weight_scale: float,
-                weight_dtype: torch.dtype) -> N.WeightJob:
-    j = N.WeightJob()
-    j.latent = latent.data_ptr()
-    j.latent_size = latent.numel()
-    j.size = int(size)
-    j.layers = int(layers)
-    j.seed = int(seed)
-    j.latent_dtype = N.dtype_code(latent.dtype)
-    j.weight_dtype = N.dtype_code(weight_dtype)
-    j.weight_scale = float(weight_scale)
-    return j
+# One lwl_bfht_weight_job (include/lwl_bfht.h): four pointers, four int64, two int32, a double and
+# an int32, packed straight into a job array (a training step packs two jobs per module; field by
+# field through ctypes each takes several times as long).
+_JOB = struct.Struct("@QQQQqqqqiidi")
+_JOB_BYTES = ctypes.sizeof(N.WeightJob)
+assert [getattr(N.WeightJob, f).offset for f, _ in N.WeightJob._fields_] == [0, 8, 16, 24, 32, 40, 48, 56, 64, 68, 72, 80]
 
 
-def _job_array(jobs: list) -> ctypes.Array:
-    return (N.WeightJob * max(1, len(jobs)))(*jobs)
+def _pack_job(arr: ctypes.Array, i: int, latent: torch.Tensor, size: int, layers: int, seed: int, weight_scale: float,
+              weight_dtype: torch.dtype, weight: int = 0, grad_weight: int = 0, grad_latent: int = 0,
+              accumulate: int = 0) -> None:
+    seed = (int(seed) + (1 << 63)) % (1 << 64) - (1 << 63)  # the int64 with the same low 64 bits
+    _JOB.pack_into(arr, i * _JOB_BYTES, latent.data_ptr(), weight, grad_weight, grad_latent, latent.numel(), int(size),
+                   int(layers), seed, N.dtype_code(latent.dtype), N.dtype_code(weight_dtype), float(weight_scale),
+                   accumulate)
+
+
+def _refused(rc: int) -> bool:
+    """A job the grouped kernels do not take (nothing was launched)."""
+    return rc in (N.LWL_ERR_INVALID, N.LWL_ERR_UNSUPPORTED)
 
 
 def weight_job_supported(latent: torch.Tensor, size: int, layers: int, weight_dtype: torch.dtype,
@@ -272,20 +277,20 @@ def weight_job_supported(latent: torch.Tensor, size: int, layers: int, weight_dt
         return False
     if not latent.is_contiguous():
         return False
-    j = _weight_job(latent, size, layers, 0, 1.0, weight_dtype)
+    arr = (N.WeightJob * 1)()
+    own = latent.data_ptr()
     if grad_weight is None:
-        j.weight = j.latent
-        forward = 1
+        _pack_job(arr, 0, latent, size, layers, 0, 1.0, weight_dtype, weight=own)
     else:
         if not grad_weight.is_cuda or not grad_weight.is_contiguous() or grad_weight.dtype != weight_dtype:
             return False
-        j.grad_weight = grad_weight.data_ptr()
-        j.grad_latent = j.latent
-        forward = 0
-    return N.lib().lwl_bfht_check_weight_jobs(_job_array([j]), 1, forward) == N.LWL_OK
+        _pack_job(arr, 0, latent, size, layers, 0, 1.0, weight_dtype, grad_weight=grad_weight.data_ptr(),
+                  grad_latent=own)
+    return N.lib().lwl_bfht_check_weight_jobs(arr, 1, int(grad_weight is None)) == N.LWL_OK
 
 
-def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = None) -> list[torch.Tensor]:
+def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = None,
+                        strict: bool = True) -> list[torch.Tensor] | None:
     """Generate whole weights of many generators in a few launches (the per-module
     ``materialize_weight_cache`` calls of the reference's ``prepare_block_fht_weight_cache``,
     ``block_fht.py:503-563``).
@@ -293,15 +298,20 @@ def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = No
     ``specs``: ``(latent, size, layers, seed, weight_scale, weight_dtype)`` per generator.
     Returns flat weights equal to ``(generate(latent) * weight_scale).to(weight_dtype)``,
     written into ``outs`` (contiguous, ``size`` elements of ``weight_dtype`` each) when given.
+    ``strict=False``: None instead of an error when the kernels do not take some generator
+    (nothing is generated then).
     """
     if not specs:
         return []
     dev = N.require_cuda(*[s[0] for s in specs])
     if outs is not None and len(outs) != len(specs):
         raise N.BlockFHTArgumentError("outs must match specs")
-    jobs, result, keep = [], [], []
+    result, keep = [], []
+    arr = (N.WeightJob * len(specs))()
     for i, (latent, size, layers, seed, weight_scale, weight_dtype) in enumerate(specs):
-        latent = latent.detach().contiguous()
+        if not latent.is_contiguous():
+            latent = latent.detach().contiguous()
+            keep.append(latent)
         if outs is None:
             out = torch.empty(int(size), dtype=weight_dtype, device=dev)
         else:
@@ -309,19 +319,18 @@ def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = No
             if (out.dtype != weight_dtype or out.numel() != int(size) or not out.is_contiguous()
                     or out.device != dev):
                 raise N.BlockFHTArgumentError(f"output {i} must be a contiguous {weight_dtype} tensor of {size}")
-        j = _weight_job(latent, size, layers, seed, weight_scale, weight_dtype)
-        j.weight = out.data_ptr()
-        jobs.append(j)
+        _pack_job(arr, i, latent, size, layers, seed, weight_scale, weight_dtype, weight=out.data_ptr())
         result.append(out)
-        keep.append(latent)
     L = N.lib()
-    arr = _job_array(jobs)
     with _device_guard(dev):
-        N.check(L.lwl_bfht_materialize_weights(arr, len(jobs), N.stream_ptr(dev)))
+        rc = L.lwl_bfht_materialize_weights(arr, len(specs), N.stream_ptr(dev))
+    if not strict and _refused(rc):
+        return None
+    N.check(rc)
     return result
 
 
-def flush_weight_grads(specs: list[tuple]) -> list[torch.Tensor]:
+def flush_weight_grads(specs: list[tuple], strict: bool = True) -> list[torch.Tensor] | None:
     """Project many weight gradients back onto their latents in a few launches (the
     per-module ``flush_weight_cache_to_latent_grad`` calls of the reference's
     ``flush_block_fht_weight_cache``, ``block_fht.py:514-569``).
@@ -330,14 +339,18 @@ def flush_weight_grads(specs: list[tuple]) -> list[torch.Tensor]:
     generator; ``into`` is None or a contiguous tensor of the latent's shape and dtype
     that the result is added to in place (``latent.grad.add_``).  Returns, per spec,
     ``into`` or a new tensor holding ``weight_scale * block_fht_grad_latent(latent,
-    grad_weight.to(latent.dtype), ...)``.
+    grad_weight.to(latent.dtype), ...)``.  ``strict=False``: None instead of an error when
+    the kernels do not take some generator (nothing is added or written then).
     """
     if not specs:
         return []
     dev = N.require_cuda(*[s[1] for s in specs])
-    jobs, outs, keep = [], [], []
-    for latent, grad_weight, size, layers, seed, weight_scale, into in specs:
-        grad_weight = grad_weight.detach().contiguous()
+    outs, keep = [], []
+    arr = (N.WeightJob * len(specs))()
+    for i, (latent, grad_weight, size, layers, seed, weight_scale, into) in enumerate(specs):
+        if not grad_weight.is_contiguous():
+            grad_weight = grad_weight.detach().contiguous()
+            keep.append(grad_weight)
         if grad_weight.numel() != size:
             raise N.BlockFHTArgumentError(f"grad_weight has {grad_weight.numel()} elements, size is {size}")
         if into is None:
@@ -346,19 +359,17 @@ def flush_weight_grads(specs: list[tuple]) -> list[torch.Tensor]:
             if into.dtype != latent.dtype or into.numel() != latent.numel() or not into.is_contiguous():
                 raise N.BlockFHTArgumentError("accumulation target must be a contiguous tensor like the latent")
             out = into
-        j = _weight_job(latent, size, layers, seed, weight_scale, grad_weight.dtype)
-        j.grad_weight = grad_weight.data_ptr()
-        j.grad_latent = out.data_ptr()
-        j.accumulate = int(into is not None)
-        jobs.append(j)
+        _pack_job(arr, i, latent, size, layers, seed, weight_scale, grad_weight.dtype,
+                  grad_weight=grad_weight.data_ptr(), grad_latent=out.data_ptr(), accumulate=int(into is not None))
         outs.append(out)
-        keep.append(grad_weight)
     L = N.lib()
-    arr = _job_array(jobs)
     with _device_guard(dev):
-        ws_ptr, ws_size, ws = N.workspace(L.lwl_bfht_flush_weight_grads_workspace_size(arr, len(jobs)), dev)
-        N.check(L.lwl_bfht_flush_weight_grads(arr, len(jobs), ws_ptr, ws_size, N.stream_ptr(dev)))
+        ws_ptr, ws_size, ws = N.workspace(L.lwl_bfht_flush_weight_grads_workspace_size(arr, len(specs)), dev)
+        rc = L.lwl_bfht_flush_weight_grads(arr, len(specs), ws_ptr, ws_size, N.stream_ptr(dev))
     del ws, keep
+    if not strict and _refused(rc):
+        return None
+    N.check(rc)
     return outs
 
 
