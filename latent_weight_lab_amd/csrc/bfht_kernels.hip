@@ -7,9 +7,9 @@
 //    slice directly; backward writes one float32 partial per block (or the
 //    final gradient when a single block is involved).
 //  * tile passes (2^16 <= B <= 2^23): the block lives in a float32 work buffer
-//    and each layer is two passes over 2^15-element LDS tiles — "low" transforms
-//    index bits 0..14 of a contiguous chunk, "high" transforms bits 15..log2(B)-1
-//    of a tile of 2^(log2B-15) rows x 2^(30-log2B) columns — so a layer costs two
+//    and each layer is two passes over 2^14-element LDS tiles — "low" transforms
+//    index bits 0..13 of a contiguous chunk, "high" transforms bits 14..log2(B)-1
+//    of a tile of 2^(log2B-14) rows x 2^(28-log2B) columns — so a layer costs two
 //    reads and two writes of the work buffer instead of one per stage.  Signs,
 //    the 1/sqrt(B) scale, zero padding, slicing and the latent/grad sources are
 //    fused into the passes' loads and stores.
@@ -340,31 +340,35 @@ __global__ __launch_bounds__(256) void bfht_sign_words_kernel(uint32_t seed32, i
 
 // ---------------------------------------------------------------- tile passes
 
-constexpr int kTileThreads = 1024;
-constexpr int kTileElems = 1 << kTileLog;
+constexpr int kPassLog = 14;            // 2^14 values per tile: two workgroups per CU
+constexpr int kPassTop = kPassLog - 5;  // the load layout's register bits start here
+constexpr int kTileThreads = 1 << kPassTop;
+constexpr int kTileElems = 1 << kPassLog;
 constexpr int kTilePadded = kTileElems + (kTileElems >> 5);
 
-// Bit groups of a tile pass that transforms tile-index bits [LO_BIT, 15): the
-// register bits of the load layout (element r * 1024 + tid holds bits 10-14
-// in r; those at or above LO_BIT, from register bit kRegLo), then [LO_BIT, 10)
-// in at most two groups of up to 5 bits from the top.
+// Bit groups of a tile pass that transforms tile-index bits [LO_BIT, 14): the
+// register bits of the load layout (element r * 512 + tid holds bits 9-13
+// in r; those at or above LO_BIT, from register bit kRegLo), then the bits below
+// them, [max(LO_BIT, 5), 9) and, in a low tile, [0, 5).
 template <int LO_BIT>
 struct TileGroups {
-  static constexpr int kRegLo = LO_BIT > 10 ? LO_BIT - 10 : 0;
-  static constexpr int kExtra = LO_BIT >= 10 ? 0 : (10 - LO_BIT + 4) / 5;
-  static constexpr int lo(int k) { return 10 - 5 * k - 5 > LO_BIT ? 10 - 5 * k - 5 : LO_BIT; }
-  static constexpr int nb(int k) { return 10 - 5 * k - lo(k); }
-  // the layout after the groups: the last extra group, or the load layout (10, 5)
-  static constexpr int kLastLo = kExtra == 0 ? 10 : lo(kExtra - 1);
+  static_assert(LO_BIT == 0 || LO_BIT >= 5, "high tiles are at least 32 columns wide");
+  static constexpr int kRegLo = LO_BIT > kPassTop ? LO_BIT - kPassTop : 0;
+  static constexpr int kExtra = LO_BIT >= kPassTop ? 0 : LO_BIT > 0 ? 1 : 2;
+  static constexpr int lo(int k) { return k > 0 ? 0 : LO_BIT > 5 ? LO_BIT : 5; }
+  static constexpr int nb(int k) { return k > 0 ? 5 : kPassTop - lo(0); }
+  // the layout after the groups: the last extra group, or the load layout (9, 5)
+  static constexpr int kLastLo = kExtra == 0 ? kPassTop : lo(kExtra - 1);
   static constexpr int kLastNb = kExtra == 0 ? 5 : nb(kExtra - 1);
 };
-static_assert(TileGroups<0>::kExtra == 2 && TileGroups<0>::lo(0) == 5 && TileGroups<0>::lo(1) == 0 &&
-                  TileGroups<0>::nb(1) == 5,
-              "low tile: bits 10-14 in registers, then 5-9 and 0-4");
-static_assert(TileGroups<7>::kExtra == 1 && TileGroups<7>::lo(0) == 7 && TileGroups<7>::nb(0) == 3,
-              "2^23 high tile: bits 10-14 in registers, then 7-9");
-static_assert(TileGroups<10>::kExtra == 0 && TileGroups<12>::kRegLo == 2, "small high tiles stay in registers");
-
+static_assert(TileGroups<0>::kExtra == 2 && TileGroups<0>::lo(0) == 5 && TileGroups<0>::nb(0) == 4 &&
+                  TileGroups<0>::lo(1) == 0 && TileGroups<0>::nb(1) == 5,
+              "low tile: bits 9-13 in registers, then 5-8 and 0-4");
+static_assert(TileGroups<8>::kExtra == 1 && TileGroups<8>::lo(0) == 8 && TileGroups<8>::nb(0) == 1,
+              "2^20 high tile: bits 9-13 in registers, then 8");
+static_assert(TileGroups<5>::kExtra == 1 && TileGroups<5>::lo(0) == 5 && TileGroups<5>::nb(0) == 4,
+              "2^23 high tile: bits 9-13 in registers, then 5-8");
+static_assert(TileGroups<9>::kExtra == 0 && TileGroups<12>::kRegLo == 3, "small high tiles stay in registers");
 
 // Sign layer in bit-group layout (L, NB): element e = group_pos(tid, r, L, NB)
 // takes bit e & 31 of table word e >> 5.
@@ -377,40 +381,40 @@ __device__ __forceinline__ void tile_signs(const uint32_t* words, float (&v)[32]
   for (int r0 = 0; r0 < 32; r0 += 8) {
 #pragma unroll
     for (int r = r0; r < r0 + 8; ++r) {
-      const int e = group_pos<kTileLog, 5>(tid, r, L, NB);
+      const int e = group_pos<kPassLog, 5>(tid, r, L, NB);
       v[r] = signed_by(v[r], words[e >> 5], e & 31);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// The same for a group below bit 10 (L >= 5): the thread's and the register's
+// The same for a group below bit 9 (L >= 5): the thread's and the register's
 // bit fields of e are disjoint and the register's lie at bit 5 and above, so
 // every register takes the same bit of the words at the thread's base plus a
 // constant per register (immediate LDS offsets, no per-register index work).
 template <int L, int NB>
 __device__ __forceinline__ void tile_signs_split(const uint32_t* words, float (&v)[32], int tid) {
   static_assert(L >= 5, "the bit within a sign word comes from the thread index alone");
-  const int e0 = group_pos<kTileLog, 5>(tid, 0, L, NB);
+  const int e0 = group_pos<kPassLog, 5>(tid, 0, L, NB);
   const uint32_t* w = words + (e0 >> 5);
   const int bit = e0 & 31;
 #pragma unroll
   for (int r0 = 0; r0 < 32; r0 += 8) {
 #pragma unroll
-    for (int r = r0; r < r0 + 8; ++r) v[r] = signed_by(v[r], w[group_pos<kTileLog, 5>(0, r, L, NB) >> 5], bit);
+    for (int r = r0; r < r0 + 8; ++r) v[r] = signed_by(v[r], w[group_pos<kPassLog, 5>(0, r, L, NB) >> 5], bit);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 // group_pos(t, r, L, NB) = group_pos(t, 0, L, NB) | group_pos(0, r, L, NB) for L >= 5, as tile_signs_split uses it
 constexpr bool tile_signs_split_ok() {
-  for (int L = 5; L <= 10; ++L)
-    for (int NB = 1; NB <= 5 && L + NB <= 15; ++NB)
+  for (int L = 5; L <= kPassTop; ++L)
+    for (int NB = 1; NB <= 5 && L + NB <= kPassLog; ++NB)
       for (int i = 0; i < 14; ++i)
         for (int r = 0; r < 32; ++r) {
           // every single thread-index bit, none, all, and two mixed patterns
-          const int t = i < 10 ? 1 << i : i == 10 ? 0 : i == 11 ? kTileThreads - 1 : i == 12 ? 0x155 : 0x2aa;
-          const int e = group_pos<kTileLog, 5>(t, r, L, NB), a = group_pos<kTileLog, 5>(t, 0, L, NB),
-                    b = group_pos<kTileLog, 5>(0, r, L, NB);
+          const int t = i < kPassTop ? 1 << i : i == 10 ? 0 : i == 11 ? kTileThreads - 1 : i == 12 ? 0x155 : 0x0aa;
+          const int e = group_pos<kPassLog, 5>(t, r, L, NB), a = group_pos<kPassLog, 5>(t, 0, L, NB),
+                    b = group_pos<kPassLog, 5>(0, r, L, NB);
           if (e != (a | b) || (a & b) != 0 || (b & 31) != 0) return false;
         }
   return true;
@@ -432,21 +436,29 @@ __device__ __forceinline__ void reg_butterflies(float (&v)[32]) {
 }
 
 
-// One pass of the tiled schedule (run_tiles).  A tile is 2^15 positions of one
+// One pass of the tiled schedule (run_tiles).  A tile is 2^14 positions of one
 // block (in registers, through LDS between bit groups): a low tile is
-// contiguous (block bits 0-14 vary), a high
-// tile is 2^(LB-15) rows of 2^(30-LB) contiguous columns, the rows walking
-// block bits 15..LB-1.  The pass loads the tile (latent, grad or the work
+// contiguous (block bits 0-13 vary), a high
+// tile is 2^(LB-14) rows of 2^(28-LB) contiguous columns, the rows walking
+// block bits 14..LB-1.  The pass loads the tile (latent, grad or the work
 // buffer), transforms its bit group (`pre`), applies the sign layer
 // `sign_layer`, transforms the same bit group again (`post`), scales, and
 // stores it (work buffer, output slice, or partial gradient row).  Each thread
-// hashes one of the tile's 1024 sign words into a shared table.  Tiles are
-// numbered slot * 2^(LB-15) + tile (2^(LB-15) tiles per block slot); the grid is
-// persistent (one workgroup per CU walks tiles blockIdx.x, + gridDim.x, ...) and
+// hashes one of the tile's 512 sign words into a shared table.  Tiles are
+// numbered slot * 2^(LB-14) + tile (2^(LB-14) tiles per block slot); the grid is
+// persistent (two workgroups per CU walk tiles blockIdx.x, + gridDim.x, ...) and
 // loads the next tile into registers while it transforms the current one, so a
 // CU's loads, transforms and stores overlap.
 //
-// Element r * 1024 + tid of the tile sits at block position pt(tid) + pr(r)
+// A pass is bound by the reads and writes of the work buffer beside the vector
+// unit's butterflies, and with one tile at a time a CU does neither during the
+// other's barriers.  So a tile takes half of a CU (66 KiB of LDS, 512 threads,
+// 128 registers each) and a second workgroup runs through them.  2^26 float32
+// values of 2^20 blocks, 3 layers: forward 343 us with tiles of 2^15 and one
+// workgroup per CU, 325 with these; backward 345, 328; 2^22 blocks 370, 322 and
+// 383, 338; one block of 2^17, 31.6 and 21.5 (twice the tiles for the idle CUs).
+//
+// Element r * 512 + tid of the tile sits at block position pt(tid) + pr(r)
 // (disjoint bit fields), so each thread keeps one 32-bit offset and adds a
 // wave-uniform one per register: the 32 loads are issued back to back without
 // per-element addresses, and range limits (latent length, slice ends) are
@@ -462,29 +474,29 @@ __device__ __forceinline__ void reg_butterflies(float (&v)[32]) {
 // workgroup, and by this one before it is written), for the block sum over
 // the groups.
 template <class T, int SRC, int DST, int TL>
-__global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
+__global__ __launch_bounds__(kTileThreads, 4) void bfht_tile_pass(
     const T* __restrict__ src_io, float* __restrict__ work, T* __restrict__ dst_io, int LB, int pre, int post,
     int n, int64_t first_block, int64_t ntiles_total, int64_t start, int64_t stop, uint32_t seed32, int sign_layer,
     float scale, int64_t group_blocks, int ngroups) {
   __shared__ float lds[kTilePadded];
   __shared__ uint32_t words[kTileElems / 32];
   static_assert(kTileElems / 32 == kTileThreads, "one sign word per thread");
-  // TL = 0: low tile; TL = LB - 15 (the launcher checks): high tile of 2^TL rows
+  // TL = 0: low tile; TL = LB - 14 (the launcher picks it): high tile of 2^TL rows
   constexpr bool high = TL > 0;
   const int tid = threadIdx.x;
-  const int tiles_log = LB - kTileLog;  // log2 tiles per block
+  const int tiles_log = LB - kPassLog;  // log2 tiles per block
   const int64_t B = (int64_t)1 << LB;
-  constexpr int col_log = kTileLog - TL;  // high tile: columns per row (>= 7 for LB <= 23)
+  constexpr int col_log = kPassLog - TL;  // high tile: columns per row (>= 5 for LB <= 23)
   constexpr int lo_bit = high ? col_log : 0;  // the tile-index bits the pass transforms
 
   // tile element e -> block position; elements 32q .. 32q+31 are positions
   // pos(32q) .. pos(32q)+31 (columns are at least 32 wide)
   auto pos = [&](uint32_t e, int tile) -> uint32_t {
-    if (!high) return ((uint32_t)tile << kTileLog) | e;
+    if (!high) return ((uint32_t)tile << kPassLog) | e;
     const uint32_t row = e >> col_log, col = e & ((1u << col_log) - 1);
-    return (row << kTileLog) | ((uint32_t)tile << col_log) | col;
+    return (row << kPassLog) | ((uint32_t)tile << col_log) | col;
   };
-  // pos(r * 1024 + tid) = pos(tid) + pr(r): the register's field does not depend on the tile
+  // pos(r * 512 + tid) = pos(tid) + pr(r): the register's field does not depend on the tile
   auto pr = [&](int r) { return (int)pos((uint32_t)r * kTileThreads, 0); };
 
   struct Geo {
@@ -536,8 +548,8 @@ __global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
   };
 
   // Bit groups (TileGroups): the load layout's register bits (element
-  // r * 1024 + tid), then the groups below bit 10 through LDS.  A tile with no
-  // group below bit 10 stays in registers from load to store.  Otherwise the
+  // r * 512 + tid), then the groups below bit 9 through LDS.  A tile with no
+  // group below bit 9 stays in registers from load to store.  Otherwise the
   // first transform starts on the loaded registers, the tile goes to LDS once
   // (freeing the registers for the next tile's loads) and visits the groups
   // downwards; the sign layer is applied in the last group's layout — for a low
@@ -548,13 +560,13 @@ __global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
   using G = TileGroups<lo_bit>;
   constexpr bool kOwnWord = G::kLastLo == 0 && G::kLastNb == 5;  // 32 consecutive positions per thread
   auto group_rw = [&](float (&v)[32], int lo, int nb, bool rd) {
-    const int b = group_base<kTileLog, 5>(tid, lo, nb);
+    const int b = group_base<kPassLog, 5>(tid, lo, nb);
     if (rd) {
 #pragma unroll
-      for (int r = 0; r < 32; ++r) v[r] = lds[group_lds<kTileLog, 5>(b, r, lo, nb)];
+      for (int r = 0; r < 32; ++r) v[r] = lds[group_lds<kPassLog, 5>(b, r, lo, nb)];
     } else {
 #pragma unroll
-      for (int r = 0; r < 32; ++r) lds[group_lds<kTileLog, 5>(b, r, lo, nb)] = v[r];
+      for (int r = 0; r < 32; ++r) lds[group_lds<kPassLog, 5>(b, r, lo, nb)] = v[r];
     }
   };
   // the tiles this workgroup walks: t0, t0 + t_step, ... below t_end
@@ -575,10 +587,11 @@ __global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
     for (int r = 0; r < 32; ++r) acc[r] = 0.0f;
   }
   // The next tile's loads are in flight during the current one's transforms,
-  // except in a summing pass over high tiles that go through LDS (blocks above
-  // 2^20): there the sum's 32 registers leave no room for them beside the
-  // transform's, and each tile is loaded at the start of its own iteration.
-  constexpr bool kPrefetch = !(DST == kDstSum && high && G::kExtra > 0);
+  // except in a summing pass over tiles that go through LDS (low tiles, and high
+  // ones of blocks above 2^19): there the sum's 32 registers leave no room for
+  // them beside the transform's, and each tile is loaded at the start of its own
+  // iteration, beside the CU's other workgroup.
+  constexpr bool kPrefetch = !(DST == kDstSum && G::kExtra > 0);
   float x[32];
   int64_t t = t0;
   if (kPrefetch && t < t_end) load_tile(geo(t), x);
@@ -595,11 +608,11 @@ __global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
       if (t + t_step < t_end) load_tile(geo(t + t_step), x);  // in flight during the transforms
       if (pre) reg_butterflies<G::kRegLo>(v);
       __syncthreads();  // the sign table is complete
-      tile_signs<10, 5>(words, v, tid);
+      tile_signs<kPassTop, 5>(words, v, tid);
       if (post) reg_butterflies<G::kRegLo>(v);
     } else {
       if (pre) reg_butterflies<G::kRegLo>(x);
-      group_rw(x, 10, 5, false);
+      group_rw(x, kPassTop, 5, false);
       if (kPrefetch && t + t_step < t_end) load_tile(geo(t + t_step), x);  // in flight during the transforms
       // downwards: the groups of the first transform (without one, straight to
       // the last group's layout), then the sign layer
@@ -619,7 +632,7 @@ __global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
 #pragma unroll
         for (int r = 0; r < 32; ++r) v[r] = signed_by(v[r], my_word, r);
       } else {
-        // a high tile's small group below bit 10.  A middle pass (work buffer to
+        // a high tile's small group below bit 9.  A middle pass (work buffer to
         // work buffer, transformed again after the signs) puts the signs on in
         // the group's layout (each element's word looked up by its tile index;
         // the table is complete: barriers since its writes).  The other passes
@@ -632,10 +645,10 @@ __global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
         } else {
           group_rw(v, G::kLastLo, G::kLastNb, false);
           __syncthreads();
-          group_rw(v, 10, 5, true);
-          tile_signs<10, 5>(words, v, tid);
+          group_rw(v, kPassTop, 5, true);
+          tile_signs<kPassTop, 5>(words, v, tid);
           if (post) {
-            group_rw(v, 10, 5, false);
+            group_rw(v, kPassTop, 5, false);
             __syncthreads();
             group_rw(v, G::kLastLo, G::kLastNb, true);
           }
@@ -654,7 +667,7 @@ __global__ __launch_bounds__(kTileThreads) void bfht_tile_pass(
           group_rw(v, G::lo(k), G::nb(k), false);
         }
         __syncthreads();
-        group_rw(v, 10, 5, true);
+        group_rw(v, kPassTop, 5, true);
         if (post) reg_butterflies<G::kRegLo>(v);
       }
     }
@@ -733,7 +746,7 @@ static hipError_t dispatch_block(int LB, bool fwd, const BfhtArgs& a, hipStream_
 template <class T, int SRC, int DST>
 static hipError_t launch_tile_kind(const BfhtArgs& a, hipStream_t s, int tl, int pre, int post, int layer,
                                    float scale, unsigned grid, int64_t group_blocks = 0, int ngroups = 0) {
-  const int64_t ntiles = a.nblocks << (a.log_block - kTileLog);
+  const int64_t ntiles = a.nblocks << (a.log_block - kPassLog);
   constexpr bool typed = SRC != kSrcWork || DST == kDstOut || DST == kDstSum;
   using U = std::conditional_t<typed, T, float>;
 #define LWL_TILE(TL)                                                                                      \
@@ -742,7 +755,6 @@ static hipError_t launch_tile_kind(const BfhtArgs& a, hipStream_t s, int tl, int
                      a.first_block, ntiles, a.start, a.stop, a.seed32, layer, scale, group_blocks, ngroups)
   switch (tl) {
     case 0: LWL_TILE(0); break;
-    case 1: if constexpr (SRC == kSrcWork) LWL_TILE(1); break;
     case 2: if constexpr (SRC == kSrcWork) LWL_TILE(2); break;
     case 3: if constexpr (SRC == kSrcWork) LWL_TILE(3); break;
     case 4: if constexpr (SRC == kSrcWork) LWL_TILE(4); break;
@@ -750,6 +762,7 @@ static hipError_t launch_tile_kind(const BfhtArgs& a, hipStream_t s, int tl, int
     case 6: if constexpr (SRC == kSrcWork) LWL_TILE(6); break;
     case 7: if constexpr (SRC == kSrcWork) LWL_TILE(7); break;
     case 8: if constexpr (SRC == kSrcWork) LWL_TILE(8); break;
+    case 9: if constexpr (SRC == kSrcWork) LWL_TILE(9); break;
     default: return hipErrorInvalidValue;
   }
 #undef LWL_TILE
@@ -766,7 +779,7 @@ static hipError_t launch_tile_pass(const BfhtArgs& a, hipStream_t s, int src, in
   return launch_tile_kind<T, kSrcWork, kDstOut>(a, s, tl, pre, post, layer, scale, grid);
 }
 
-// Blocks above 2^15: H = H_low (x) H_high over block bits 0-14 and 15..LB-1,
+// Blocks above 2^15: H = H_low (x) H_high over block bits 0-13 and 14..LB-1,
 // the two factors commute, so consecutive layers share a pass:
 //   [D_0, H_low] [H_high, D_1, H_high] [H_low, D_2, H_low] ... [H_g, D_L, out]
 // (L + 1 passes, each one read and one write of the float32 work buffer).
@@ -774,9 +787,9 @@ static hipError_t launch_tile_pass(const BfhtArgs& a, hipStream_t s, int src, in
 // runs the same schedule on grad with the sign layers in reverse (D_L first,
 // D_0 last); its last pass (kDstSum) also sums the blocks: each workgroup adds
 // one tile position range over a group of blocks, with enough groups to give
-// every CU a workgroup, and only with more than one group does a block sum
-// over the groups' rows follow (config 3: 2^20 blocks, 64 blocks in 8 groups,
-// 32 MiB of rows instead of 256 MiB; 2^23, 8 blocks in one group, no rows).
+// every CU its two workgroups, and only with more than one group does a block sum
+// over the groups' rows follow (64 blocks of 2^20 in 8 groups, 32 MiB of rows
+// instead of 256 MiB; 8 of 2^23 in one group, no rows).
 // The CU count of the current device, cached per device: each slot is written
 // with the same value by whichever thread gets there first (relaxed atomics,
 // so concurrent callers need no lock).
@@ -797,9 +810,9 @@ int64_t device_cus() {
   return cus;
 }
 
-// Workgroups of the persistent tile passes: one per CU (a workgroup takes all
-// of a CU's LDS), never more than the tiles.
-static unsigned tile_grid(int64_t ntiles) { return (unsigned)std::min<int64_t>(ntiles, device_cus()); }
+// Workgroups of the persistent tile passes: two per CU (a workgroup takes just
+// under half of a CU's LDS), never more than the tiles.
+static unsigned tile_grid(int64_t ntiles) { return (unsigned)std::min<int64_t>(ntiles, 2 * device_cus()); }
 
 template <class T>
 static hipError_t run_tiles(const BfhtArgs& a, hipStream_t s, bool fwd);
@@ -826,21 +839,21 @@ static hipError_t run_tiles_grouped(const BfhtArgs& a, hipStream_t s) {
 
 template <class T>
 static hipError_t run_tiles(const BfhtArgs& a, hipStream_t s, bool fwd) {
-  const int64_t tiles_per_block = (int64_t)1 << (a.log_block - kTileLog);
+  const int64_t tiles_per_block = (int64_t)1 << (a.log_block - kPassLog);
   const unsigned grid = tile_grid(a.nblocks * tiles_per_block);
   const int L = a.layers;
   const int LB = a.log_block;
   const float norm = (LB & 1) ? 0.70710678118654752440f / (float)(1 << (LB >> 1)) : 1.0f / (float)(1 << (LB >> 1));
   // the backward's summing last pass: groups of group_blocks blocks, one
-  // workgroup per (tile, group), at least as many workgroups as CUs where the
+  // workgroup per (tile, group), at least two workgroups per CU where the
   // blocks allow, no empty group
-  const int64_t cus = device_cus();
-  int64_t ngroups = std::min<int64_t>(std::max<int64_t>((cus + tiles_per_block - 1) / tiles_per_block, 1), a.nblocks);
+  const int64_t wgs = 2 * device_cus();
+  int64_t ngroups = std::min<int64_t>(std::max<int64_t>((wgs + tiles_per_block - 1) / tiles_per_block, 1), a.nblocks);
   const int64_t group_blocks = (a.nblocks + ngroups - 1) / ngroups;
   ngroups = (a.nblocks + group_blocks - 1) / group_blocks;
   for (int k = 0; k <= L; ++k) {
     const int src = k == 0 ? (fwd ? kSrcLatent : kSrcGrad) : kSrcWork;
-    const int tl = (k & 1) ? LB - kTileLog : 0;  // odd passes run high tiles
+    const int tl = (k & 1) ? LB - kPassLog : 0;  // odd passes run high tiles
     const float scale = k > 0 ? norm : 1.0f;
     hipError_t e;
     if (k == L && !fwd)

@@ -16,10 +16,11 @@ constexpr int kWholeBlockMaxLog = 15;
 
 // The tile-pass forward runs its passes over groups of blocks whose work
 // buffer is at most 128 MiB (at least one block): a group's passes then find
-// more of the buffer in the 256 MB last-level cache (config 3, 2^26
+// more of the buffer in the 256 MB last-level cache (float32, 3 layers, 2^26
 // coordinates in two groups, same box: 0.421 -> 0.397-0.403 ms at 2^23
 // blocks, 2^20 unchanged within the spread), the workspace halves, and
-// quarter-size groups leave too few tiles per CU (0.42 / 0.44 ms).  The
+// groups of half that size leave too few tiles per CU (2^20 blocks 325 -> 363 us,
+// 2^23 354 -> 389).  The
 // backward, whose last pass sums across blocks, does not gain and is not split.
 constexpr int64_t kTileGroupBytes = (int64_t)128 << 20;
 inline int64_t tile_group_blocks(int log_block) {

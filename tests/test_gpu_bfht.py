@@ -366,3 +366,23 @@ def test_reference_2_23_smoke():
     lat = bfht.latent.detach().double().cpu().numpy()
     want = c_oracle.forward(lat, 1 << 23, 1, 9, 12345, 12345 + 1024)
     assert rel_l2(to_np(out), want) < 1e-5
+
+
+@pytest.mark.parametrize("log_block,nblocks,layers,dtype", [
+    (23, 2, 1, torch.float32),      # 512 tiles per block: one group of two blocks, summed straight into grad_latent
+    (16, 301, 2, torch.float16),    # even L: low tiles in the summing pass, 101 groups of 3 blocks
+    (19, 33, 3, torch.float32),     # 512 columns: the largest block whose high tiles stay in registers
+    (20, 9, 1, torch.bfloat16),     # one bit of the high tile below the registers
+])
+def test_half_cu_tiles(log_block, nblocks, layers, dtype):
+    """Tiles of 2^14, two workgroups per CU: the block sum with one group and with low tiles
+    in its pass, and both sides of the register-only high tiles, forward and backward."""
+    B = 1 << log_block
+    n = B - 5
+    size = nblocks * B - 11
+    lat = latent_for(n, nblocks, dtype)
+    y = ops.forward(lat.cuda(), size, layers, 31, 0, size)
+    assert rel_l2(to_np(y), c_oracle.forward(lat.double().numpy(), size, layers, 31, 0, size)) < TOL[dtype]
+    g = torch.randn(size, generator=torch.Generator().manual_seed(nblocks)).to(dtype)
+    gl = ops.backward(g.cuda(), n, dtype, size, layers, 31, 0, size)
+    assert rel_l2(to_np(gl), c_oracle.backward(g.double().numpy(), n, size, layers, 31, 0, size)) < TOL[dtype]
