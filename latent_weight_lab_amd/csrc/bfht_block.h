@@ -111,28 +111,10 @@ __device__ __forceinline__ void block_fwd_small(const T* __restrict__ latent, St
     if (r >= lo && r < hi) out.at(base + r - start, v[r]);
 }
 
-template <int LB, class T, class Load>
-__device__ __forceinline__ void block_bwd_small(Load grad, float* __restrict__ partial, int64_t stride,
-                                                T* __restrict__ grad_latent, int n, int64_t first_block, int64_t slot,
-                                                int64_t nblocks, int64_t start, int64_t stop, uint32_t seed32,
-                                                int layers, int direct) {
+// The adjoint chain D_0 H D_1 ... H D_L of one thread's block.
+template <int LB>
+__device__ __forceinline__ void block_bwd_small_layers(float (&v)[Geo<LB>::E], uint32_t bkey, int layers) {
   using Gm = Geo<LB>;
-  static_assert(Gm::TB == 1, "one thread per block");
-  const bool active = slot < nblocks;
-  const int64_t block = first_block + (active ? slot : 0);
-  const uint32_t bkey = block_key(seed32, block);
-  const int64_t base = block * Gm::B;
-  const int64_t lo = start - base > 0 ? start - base : 0;
-  const int64_t hi = stop - base < Gm::B ? stop - base : Gm::B;
-  // every lane is a different block: element loads from a valid index (the
-  // slice's first element stands in for positions outside it), then a select
-  float v[Gm::E];
-#pragma unroll
-  for (int r = 0; r < Gm::E; ++r) {
-    const bool valid = active && r >= lo && r < hi;
-    const float x = grad.at(valid ? base + r - start : 0);
-    v[r] = valid ? x : 0.0f;
-  }
   const float scale = inv_sqrt_block<LB>();
   for (int layer = layers - 1; layer >= 0; --layer) {
     const uint32_t w = sign_word(bkey, layer_key(layer + 1), 0u);
@@ -142,18 +124,9 @@ __device__ __forceinline__ void block_bwd_small(Load grad, float* __restrict__ p
 #pragma unroll
     for (int r = 0; r < Gm::E; ++r) v[r] *= scale;
   }
-  if (!active) return;
   const uint32_t w0 = sign_word(bkey, layer_key(0), 0u);
 #pragma unroll
-  for (int r = 0; r < Gm::E; ++r) {
-    if (r < n) {
-      const float g = signed_by(v[r], w0, r);
-      if (direct)
-        grad_latent[r] = from_f32<T>(g);
-      else
-        partial[slot * stride + r] = g;
-    }
-  }
+  for (int r = 0; r < Gm::E; ++r) v[r] = signed_by(v[r], w0, r);
 }
 
 // Layout of bit group [lo, lo + nb) (nb <= 5) in the whole-block kernels:
@@ -432,101 +405,168 @@ __device__ __forceinline__ void block_fwd_slot(const T* __restrict__ latent, Sto
   }
 }
 
-// Backward: adjoint chain D_0 H D_1 ... H D_L on grad scattered into the block.
-// Writes partial[slot * stride + p] (float32) for p < n, or the final gradient
-// in T when `direct` (a single block).
-template <int LB, class T, class Load>
-__device__ __forceinline__ void block_bwd_slot(Load grad, float* __restrict__ partial, int64_t stride,
-                                               T* __restrict__ grad_latent, int n, int64_t first_block, int64_t slot,
-                                               int64_t nblocks, int64_t start, int64_t stop, uint32_t seed32,
-                                               int layers, int direct, float* smem) {
+// The adjoint chain D_0 H D_1 ... H D_L without its scale: v enters in the
+// coalesced layout and leaves in the layout of group 0 (even layer counts) or of
+// the last group (odd).  `table`: word index of the block's sign table.
+template <int LB>
+__device__ __forceinline__ void block_bwd_layers(float (&v)[32], float* lds, const uint32_t* words, int table, int t,
+                                                 int layers) {
   using Gm = Geo<LB>;
   using S = BlockSeq<LB>;
-  if constexpr (Gm::NG <= 1) {  // B <= 2^5
-    block_bwd_small<LB, T>(grad, partial, stride, grad_latent, n, first_block, slot, nblocks, start, stop, seed32,
-                           layers, direct);
-  } else {
-    const int gi = threadIdx.x >> Gm::LT;
-    const int t = threadIdx.x & (Gm::TB - 1);
-    const bool active = slot < nblocks;
-    const int64_t block = first_block + (active ? slot : 0);
-    float* lds = BlockLds<LB>::data(smem, gi);
-    uint32_t* tab = BlockLds<LB>::table(smem, gi);
-    fill_sign_table<LB>(tab, block_key(seed32, block), t, layers);
-    const int64_t base = block * Gm::B;
-    const int64_t lo = start - base > 0 ? start - base : 0;
-    const int64_t hi = stop - base < Gm::B ? stop - base : Gm::B;
-    // positions outside [lo, hi), and every position of an inactive slot, read 0
-    float v[32];
-    if constexpr (Gm::TB >= 64) {
-      const auto g_r = grad.range(base + lo - start, active ? hi - lo : 0);
-      if (active && lo == 0 && hi == Gm::B) {  // a whole block: no per-element checks
+  sign_flip<LB>(v, words, table + layers * Gm::TB, t, S::lo(0), S::nb(0));
+  for (int i = 0; i < layers; ++i) {
+    const bool odd = i & 1;
+    layer_fht<LB>(v, lds, t, odd);
+    const int lw = table + (layers - 1 - i) * Gm::TB;
+    if (odd)
+      sign_flip<LB>(v, words, lw, t, S::lo(0), S::nb(0));
+    else
+      sign_flip<LB>(v, words, lw, t, S::lo(S::N - 1), S::nb(S::N - 1));
+  }
+}
+
+// LDS of the backward: the transform's, or every thread group's summed block.
+template <int LB>
+struct BwdLds {
+  using Gm = Geo<LB>;
+  static constexpr int kSum = Gm::G * Gm::PADDED;  // padded rows; at least the 256 chunk sums
+  static constexpr int kMost = BlockLds<LB>::FLOATS > kSum ? BlockLds<LB>::FLOATS : kSum;
+  static constexpr int FLOATS = kMost > 256 ? kMost : 256;
+};
+
+template <int LB>
+inline constexpr bool kBwdSingle = Geo<LB>::G == 1 && Geo<LB>::WG < 1024;  // has a kLoop = false variant
+
+// Backward of whole blocks: the adjoint chain D_0 H D_1 ... H D_L on grad scattered
+// into each block, summed over a run of blocks.  A workgroup takes the G blocks
+// (one per thread group) of `run` consecutive ranges from range `index` * run on,
+// one range after another, adds every thread's scaled result up in registers, adds
+// the thread groups up through LDS, and writes one row: row[p] (float32, p < n), or
+// the gradient itself (grad_latent set: the call's only row).  Fixed order throughout.
+//
+// A row per block costs a float32 write and read of the whole slice beside the
+// gradient's read, and the block sum of a short latent has thousands of rows per
+// column and a few columns to share between workgroups.  float32, 2^25 values:
+// latent 2^15, 96 -> 69 us (now bound by the vector unit's butterflies, as the
+// forward is); 2^12, 98 -> 55; 2^10, 231 -> 38; 2^6, 3040 -> 79.  A latent of 1000
+// under 4000 values: one row, so no second launch, 10.2 -> 6.9 us.
+// kLoop = false (2^13 and 2^14, one block per workgroup): no sum, no registers
+// for it (2^14 under 2^22 values took 18.7 us with them, 16.7 without; at 2^15
+// it made no difference).
+template <int LB, class T, bool kLoop, class Load>
+__device__ __forceinline__ void block_bwd_row(Load grad, float* __restrict__ row, T* __restrict__ grad_latent, int n,
+                                              int64_t first_block, int64_t index, int run, int64_t start,
+                                              int64_t stop, uint32_t seed32, int layers, float* smem) {
+  using Gm = Geo<LB>;
+  using S = BlockSeq<LB>;
+  constexpr int E = Gm::E, B = Gm::B, G = Gm::G, TB = Gm::TB;
+  constexpr int kRange = G * B;  // positions of one range
+  const int gi = threadIdx.x >> Gm::LT;
+  const int t = threadIdx.x & (TB - 1);
+  float acc[E];
 #pragma unroll
-        for (int r = 0; r < 32; ++r) v[r] = grad.whole(g_r, t, r * Gm::TB);
-      } else {
+  for (int r = 0; r < E; ++r) acc[r] = 0.0f;
+  for (int k = 0; k < (kLoop ? run : 1); ++k) {
+    // The range as one buffer: blocks past the slice's end, and positions outside
+    // it, read 0 and add 0.
+    const int64_t b0 = first_block + (index * run + k) * G;
+    const int64_t base = b0 * B;
+    const int lo = start > base ? (int)(start - base) : 0;  // start lies in the first range
+    const int64_t left = stop - base;
+    const int hi = left < 0 ? 0 : left < kRange ? (int)left : kRange;
+    const auto g_r = grad.range(base + lo - start, hi > lo ? hi - lo : 0);
+    const int p0 = gi * B + t;
+    float v[E];
+    if (lo == 0 && hi == kRange) {  // a whole range: no per-element checks
 #pragma unroll
-        for (int r = 0; r < 32; ++r) v[r] = grad(g_r, r * Gm::TB + t - (int)lo);
-      }
+      for (int r = 0; r < E; ++r) v[r] = grad.whole(g_r, p0, r * TB);
     } else {
-      // several blocks per wave: element loads from a valid index (the slice's
-      // first element stands in for positions outside it), then a select
+#pragma unroll
+      for (int r = 0; r < E; ++r) v[r] = grad(g_r, p0 + r * TB - lo);
+    }
+    const uint32_t bkey = block_key(seed32, b0 + gi);
+    if constexpr (Gm::NG <= 1) {
+      block_bwd_small_layers<LB>(v, bkey, layers);
+#pragma unroll
+      for (int r = 0; r < E; ++r) acc[r] += v[r];
+    } else {
+      if (k > 0) __syncthreads();  // the previous range's reads of the table and the exchange buffers are done
+      fill_sign_table<LB>(BlockLds<LB>::table(smem, gi), bkey, t, layers);
+      __syncthreads();  // the sign table is complete
+      block_bwd_layers<LB>(v, BlockLds<LB>::data(smem, gi), reinterpret_cast<const uint32_t*>(smem),
+                           BlockLds<LB>::table_word(gi), t, layers);
+      const float scale = transform_scale<LB>(layers);
+#pragma unroll
+      for (int r = 0; r < E; ++r) acc[r] = kLoop ? acc[r] + v[r] * scale : v[r] * scale;
+    }
+  }
+  if constexpr (G == 1) {
+    static_assert(S::kLastStores, "the last group's layout stores 32 consecutive positions per half wave");
+    auto write = [&](int glo, int gnb) {
+      const int pb = bpos<LB>(t, 0, glo, gnb);
+      // positions >= n dropped
+      const auto d_r = grad_latent ? tile_rsrc(grad_latent, (uint64_t)n * sizeof(T)) : tile_rsrc(row, (uint64_t)n * 4);
 #pragma unroll
       for (int r = 0; r < 32; ++r) {
-        const int p = r * Gm::TB + t;
-        const bool valid = active && p >= lo && p < hi;
-        const float x = grad.at(valid ? base + p - start : 0);
-        v[r] = valid ? x : 0.0f;
-      }
-    }
-    __syncthreads();  // the sign table is complete
-    const uint32_t* words = reinterpret_cast<const uint32_t*>(smem);
-    const int tw = BlockLds<LB>::table_word(gi);
-    sign_flip<LB>(v, words, tw + layers * Gm::TB, t, S::lo(0), S::nb(0));
-    for (int i = 0; i < layers; ++i) {
-      const bool odd = i & 1;
-      layer_fht<LB>(v, lds, t, odd);
-      const int lw = tw + (layers - 1 - i) * Gm::TB;
-      if (odd)
-        sign_flip<LB>(v, words, lw, t, S::lo(0), S::nb(0));
-      else
-        sign_flip<LB>(v, words, lw, t, S::lo(S::N - 1), S::nb(S::N - 1));
-    }
-    const float scale = transform_scale<LB>(layers);
-    auto write = [&](int glo, int gnb) {
-      if (!active) return;
-      const int pb = bpos<LB>(t, 0, glo, gnb);
-      if constexpr (Gm::TB >= 64) {
-        // one block per wave: uniform resources, positions >= n dropped
-        const auto d_r = direct ? tile_rsrc(grad_latent, (uint64_t)n * sizeof(T))
-                                : tile_rsrc(partial + slot * stride, (uint64_t)n * 4);
-#pragma unroll
-        for (int r = 0; r < 32; ++r) {
-          const int c = bpos<LB>(0, r, glo, gnb);  // disjoint from pb's bits
-          if (direct)
-            buf_store_nn<T>(v[r] * scale, d_r, pb, c);
-          else
-            buf_store_nn<float>(v[r] * scale, d_r, pb, c);
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 32; ++r) {
-          const int p = pb | bpos<LB>(0, r, glo, gnb);
-          if (p < n) {
-            if (direct)
-              grad_latent[p] = from_f32<T>(v[r] * scale);
-            else
-              partial[slot * stride + p] = v[r] * scale;
-          }
-        }
+        const int c = bpos<LB>(0, r, glo, gnb);  // disjoint from pb's bits
+        if (grad_latent)
+          buf_store_nn<T>(acc[r], d_r, pb, c);
+        else
+          buf_store_nn<float>(acc[r], d_r, pb, c);
       }
     };
-    if (!(layers & 1)) {
-      write(S::lo(0), S::nb(0));
-    } else if constexpr (S::kLastStores) {
+    if (layers & 1)
       write(S::lo(S::N - 1), S::nb(S::N - 1));
-    } else {
-      exchange<LB>(v, lds, t, S::lo(S::N - 1), S::nb(S::N - 1), S::lo(0), S::nb(0), Gm::TB <= 64);
+    else
       write(S::lo(0), S::nb(0));
+  } else {
+    float* mine = smem + gi * Gm::PADDED;
+    if constexpr (Gm::NG <= 1) {
+#pragma unroll
+      for (int r = 0; r < E; ++r) mine[r] = acc[r];
+    } else {
+      __syncthreads();  // the exchange buffers are no longer read
+      auto put = [&](int glo, int gnb) {
+        const int b = bslot_base<LB>(t, glo, gnb);
+#pragma unroll
+        for (int r = 0; r < 32; ++r) mine[bslot<LB>(b, r, glo, gnb)] = acc[r];
+      };
+      if (layers & 1)
+        put(S::lo(S::N - 1), S::nb(S::N - 1));
+      else
+        put(S::lo(0), S::nb(0));
+    }
+    __syncthreads();
+    // Position p of every thread group: below 256 positions the 256 threads
+    // split the groups into chunks, whose sums are added in a second step.
+    static_assert(Gm::WG == 256, "several blocks per workgroup of 256 threads");
+    constexpr int kCols = B < 256 ? B : 256;
+    constexpr int kChunks = 256 / kCols, kPer = G / kChunks;
+    const int tid = threadIdx.x, c = tid / kCols;
+    auto write = [&](int p, float s) {
+      if (p >= n) return;
+      if (grad_latent)
+        grad_latent[p] = from_f32<T>(s);
+      else
+        row[p] = s;
+    };
+#pragma unroll 1
+    for (int p = tid & (kCols - 1); p < B; p += kCols) {
+      float s = 0.0f;
+#pragma unroll 8
+      for (int j = 0; j < kPer; ++j) s += smem[(c * kPer + j) * Gm::PADDED + lds_index(p)];
+      if constexpr (kChunks == 1) {
+        write(p, s);
+      } else {  // B = kCols: every thread comes here once
+        __syncthreads();
+        smem[tid] = s;
+        __syncthreads();
+        if (tid < B) {
+          float total = 0.0f;
+          for (int q = 0; q < kChunks; ++q) total += smem[q * kCols + tid];
+          write(tid, total);
+        }
+      }
     }
   }
 }

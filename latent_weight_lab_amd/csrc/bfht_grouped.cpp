@@ -36,9 +36,10 @@ struct ClassKey {
   int wdtype;  // VALU classes only (a template parameter there)
   int log_block;
   int layers;  // matrix-core classes only (a template parameter there)
+  bool summed = false;  // matrix-core backward of several blocks per row (its own kernel)
   bool operator==(const ClassKey& o) const {
     return mfma == o.mfma && dtype == o.dtype && wdtype == o.wdtype && log_block == o.log_block &&
-           layers == o.layers;
+           layers == o.layers && summed == o.summed;
   }
 };
 
@@ -87,6 +88,12 @@ GroupJob device_job(const WeightJob& j, bool fwd, void* part) {
   d.stride = (int32_t)row_stride(j);
   d.part_bf16 = !fwd && part_bf16(j);
   d.nblocks = (int32_t)blocks_of(j);
+  if (!fwd) {
+    const int lb = log2_ceil(j.n);
+    const bool mfma = d.part_bf16 != 0;
+    d.run = (int32_t)(mfma ? mfma15_bwd_group(d.nblocks) : block_bwd_run(lb, d.nblocks));
+    d.rows = (int32_t)(mfma ? mfma15_bwd_rows(d.nblocks) : block_bwd_rows(lb, d.nblocks));
+  }
   d.seed32 = j.seed32;
   d.layers = j.layers;
   d.wdtype = j.wdtype;
@@ -156,6 +163,7 @@ hipError_t launch_grouped(const WeightJob* jobs, int64_t count, void* work, hipS
     }
     djobs[i] = device_job(jobs[i], fwd, part);
     keys[i] = class_of(jobs[i], fwd);
+    keys[i].summed = keys[i].mfma && djobs[i].run > 1;
   }
   // classes in order of first appearance
   std::vector<bool> done((size_t)count, false);
@@ -169,9 +177,9 @@ hipError_t launch_grouped(const WeightJob* jobs, int64_t count, void* work, hipS
         done[m] = true;
       }
     const hipError_t e = run_tables(
-        idx, djobs, [&](int m) { return workgroups_of(k, jobs[m]); },
+        idx, djobs, [&](int m) { return fwd ? workgroups_of(k, jobs[m]) : (int64_t)djobs[m].rows; },
         [&](const GroupTable& t) {
-          return k.mfma ? launch_mfma15_grouped(t, k.layers, s, fwd)
+          return k.mfma ? launch_mfma15_grouped(t, k.layers, s, fwd, k.summed)
                         : launch_block_grouped(t, k.dtype, k.wdtype, k.log_block, s, fwd);
         });
     if (e != hipSuccess) return e;

@@ -41,7 +41,6 @@ struct WeightGradLoad {
   __device__ float whole(__amdgpu_buffer_rsrc_t r, int base, int c) const {
     return round_to<T>(buf_load_at<W>(r, base, c));
   }
-  __device__ float at(int64_t i) const { return round_to<T>(to_f32(g[i])); }
 };
 
 template <int LB, class T, class W>
@@ -54,25 +53,29 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_block_fwd_grouped(const Grou
                         0, slot, jb.nblocks, 0, jb.size, jb.seed32, jb.layers, smem);
 }
 
-template <int LB, class T, class W>
-__global__ __launch_bounds__(Geo<LB>::WG) void bfht_block_bwd_grouped(const GroupTable g) {
-  __shared__ float smem[BlockLds<LB>::FLOATS];
+template <int LB, class T, class W, bool kLoop>
+__global__ __launch_bounds__(Geo<LB>::WG, 4) void bfht_block_bwd_grouped(const GroupTable g) {
+  __shared__ float smem[BwdLds<LB>::FLOATS];
   const int j = group_job(g, (int)blockIdx.x);
   const GroupJob& jb = g.job[j];
-  const int64_t slot = (int64_t)(blockIdx.x - g.prefix[j]) * Geo<LB>::G + (threadIdx.x >> Geo<LB>::LT);
-  block_bwd_slot<LB, T>(WeightGradLoad<T, W>{static_cast<const W*>(jb.src)}, static_cast<float*>(jb.part), jb.stride,
-                        static_cast<T*>(nullptr), jb.n, 0, slot, jb.nblocks, 0, jb.size, jb.seed32, jb.layers, 0,
-                        smem);
+  const int64_t index = (int64_t)blockIdx.x - g.prefix[j];
+  block_bwd_row<LB, T, kLoop>(WeightGradLoad<T, W>{static_cast<const W*>(jb.src)},
+                              static_cast<float*>(jb.part) + index * jb.stride, static_cast<T*>(nullptr), jb.n, 0,
+                              index, jb.run, 0, jb.size, jb.seed32, jb.layers, smem);
 }
 
 template <int LB, class T, class W>
 hipError_t launch_lb(const GroupTable& g, hipStream_t s, bool fwd) {
   if (group_slots_per_wg(LB) != Geo<LB>::G) return hipErrorInvalidValue;  // the planner's prefix unit
   const dim3 grid((unsigned)g.prefix[g.count]), block(Geo<LB>::WG);
+  bool loop = !kBwdSingle<LB>;
+  for (int j = 0; j < g.count; ++j) loop = loop || g.job[j].run > 1;
   if (fwd)
     hipLaunchKernelGGL((bfht_block_fwd_grouped<LB, T, W>), grid, block, 0, s, g);
+  else if (loop)
+    hipLaunchKernelGGL((bfht_block_bwd_grouped<LB, T, W, true>), grid, block, 0, s, g);
   else
-    hipLaunchKernelGGL((bfht_block_bwd_grouped<LB, T, W>), grid, block, 0, s, g);
+    hipLaunchKernelGGL((bfht_block_bwd_grouped<LB, T, W, !kBwdSingle<LB>>), grid, block, 0, s, g);
   return hipGetLastError();
 }
 

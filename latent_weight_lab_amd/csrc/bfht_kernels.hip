@@ -4,8 +4,8 @@
 //  * whole-block kernels (B <= 2^15): one block per workgroup slot, resident
 //    in VGPRs (32 per thread) with LDS exchanges, all layers in one launch;
 //    small blocks pack several per workgroup.  Forward writes the requested
-//    slice directly; backward writes one float32 partial per block (or the
-//    final gradient when a single block is involved).
+//    slice directly; backward writes one float32 row per workgroup, the sum of
+//    its blocks (or the final gradient when one workgroup has them all).
 //  * tile passes (2^16 <= B <= 2^23): the block lives in a float32 work buffer
 //    and each layer is two passes over 2^14-element LDS tiles — "low" transforms
 //    index bits 0..13 of a contiguous chunk, "high" transforms bits 14..log2(B)-1
@@ -24,10 +24,9 @@
 
 namespace lwl {
 
-// Element access of the per-generator launches: the slice in the latent dtype.
 // Element access of the per-generator launches: the slice in the latent dtype,
-// through a buffer resource over one block's range (`range` + call) or by
-// element index (`at`, for blocks that share a wave).
+// through a buffer resource over a range of it (`range` + call) or, in the
+// forward, by element index (`at`, for blocks that share a wave).
 template <class T>
 struct SliceStore {
   T* out;
@@ -46,7 +45,6 @@ struct SliceLoad {
   }
   __device__ float operator()(__amdgpu_buffer_rsrc_t r, int i) const { return buf_load<T>(r, i); }
   __device__ float whole(__amdgpu_buffer_rsrc_t r, int base, int c) const { return buf_load_at<T>(r, base, c); }
-  __device__ float at(int64_t i) const { return to_f32(g[i]); }
 };
 
 template <int LB, class T>
@@ -60,17 +58,15 @@ __global__ __launch_bounds__(Geo<LB>::WG) void bfht_block_fwd(const T* __restric
                         smem);
 }
 
-template <int LB, class T>
-__global__ __launch_bounds__(Geo<LB>::WG) void bfht_block_bwd(const T* __restrict__ grad,
-                                                             float* __restrict__ partial,
-                                                             T* __restrict__ grad_latent, int n,
-                                                             int64_t first_block, int64_t nblocks, int64_t start,
-                                                             int64_t stop, uint32_t seed32, int layers,
-                                                             int direct) {
-  __shared__ float smem[BlockLds<LB>::FLOATS];
-  const int64_t slot = (int64_t)blockIdx.x * Geo<LB>::G + (threadIdx.x >> Geo<LB>::LT);
-  block_bwd_slot<LB, T>(SliceLoad<T>{grad}, partial, n, grad_latent, n, first_block, slot, nblocks, start, stop,
-                        seed32, layers, direct, smem);
+template <int LB, class T, bool kLoop>
+__global__ __launch_bounds__(Geo<LB>::WG, 4) void bfht_block_bwd(const T* __restrict__ grad,
+                                                                float* __restrict__ partial,
+                                                                T* __restrict__ grad_latent, int n,
+                                                                int64_t first_block, int64_t start, int64_t stop,
+                                                                uint32_t seed32, int layers, int run, int direct) {
+  __shared__ float smem[BwdLds<LB>::FLOATS];
+  block_bwd_row<LB, T, kLoop>(SliceLoad<T>{grad}, partial + (int64_t)blockIdx.x * n, direct ? grad_latent : nullptr, n,
+                              first_block, blockIdx.x, run, start, stop, seed32, layers, smem);
 }
 
 // grad_latent[p] = sum_b part[b * stride + p], blocks in order.
@@ -265,7 +261,7 @@ __global__ __launch_bounds__(64 * kRedWaves) void bfht_reduce_grouped(const Grou
   const int n = jb.n;
   const int c0 = ((blockIdx.x - g.prefix[j]) * 64 + (threadIdx.x & 63)) * 4;
   float t[4];
-  if (!reduce_columns<4, P>(static_cast<const P*>(jb.part), jb.nblocks, jb.stride, n, c0, sums, t)) return;
+  if (!reduce_columns<4, P>(static_cast<const P*>(jb.part), jb.rows, jb.stride, n, c0, sums, t)) return;
   T* dst = static_cast<T*>(jb.dst);
   // an accumulating job reads its four destination values together first
   // (each read behind its own column check was waited out on its own)
@@ -720,14 +716,15 @@ static hipError_t launch_block_fwd(const BfhtArgs& a, hipStream_t s) {
 template <int LB, class T>
 static hipError_t launch_block_bwd(const BfhtArgs& a, hipStream_t s) {
   using Gm = Geo<LB>;
-  const int64_t grid = (a.nblocks + Gm::G - 1) / Gm::G;
-  const int direct = a.nblocks == 1;
-  hipLaunchKernelGGL((bfht_block_bwd<LB, T>), dim3((unsigned)grid), dim3(Gm::WG), 0, s,
-                     (const T*)a.src, (float*)a.work, (T*)a.dst, (int)a.n, a.first_block,
-                     a.nblocks, a.start, a.stop, a.seed32, a.layers, direct);
+  const int64_t run = block_bwd_run(LB, a.nblocks), rows = block_bwd_rows(LB, a.nblocks);
+  const int direct = rows == 1;
+  const auto kernel =
+      kBwdSingle<LB> && run == 1 ? &bfht_block_bwd<LB, T, !kBwdSingle<LB>> : &bfht_block_bwd<LB, T, true>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(Gm::WG), 0, s, (const T*)a.src, (float*)a.work, (T*)a.dst,
+                     (int)a.n, a.first_block, a.start, a.stop, a.seed32, a.layers, (int)run, direct);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || direct) return e;
-  return launch_reduce<T>((const float*)a.work, a.nblocks, a.n, a.n, (T*)a.dst, s);
+  return launch_reduce<T>((const float*)a.work, rows, a.n, a.n, (T*)a.dst, s);
 }
 
 template <class T>

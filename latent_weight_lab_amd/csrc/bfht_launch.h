@@ -66,12 +66,31 @@ inline bool chains_share_cu(int64_t blocks) { return blocks > device_cus(); }
 void* noalloc_scratch(hipStream_t s, hipError_t* err);
 
 // Matrix-core path for bfloat16 blocks of exactly 2^15 (bfht_mfma.hip).  The
-// backward writes one float32 partial row of n values per block into `work`.
+// backward writes mfma15_bwd_rows bfloat16 partial rows into `work`.
 bool mfma15_applicable(const BfhtArgs& a, bool fwd);
 // The matrix-core backward's partial rows: bfloat16, rows of n padded to 8
 // elements (16-byte aligned), inside the float32-row workspace.
 __host__ __device__ inline int64_t mfma15_part_stride(int64_t n) { return (n + 7) / 8 * 8; }
 hipError_t launch_mfma15(const BfhtArgs& a, hipStream_t s, bool forward);
+// Blocks of 2^log_block <= 2^15 that one workgroup transforms together (Geo::G).
+int group_slots_per_wg(int log_block);
+// The vector-unit backward of nblocks whole blocks: ranges of group_slots_per_wg
+// blocks that one workgroup adds up, and the rows it leaves.  One range while the
+// chip holds them all at once (1024 threads per CU), beyond that the fewest that make
+// one such set.  Where several workgroups share a CU, only from two sets on: between
+// one and two, two ranges each leave CUs half empty (513 blocks of 2^14: 30.6 us
+// against 28.0 with a row per block).
+inline int64_t block_bwd_run(int log_block, int64_t nblocks) {
+  const int64_t g = group_slots_per_wg(log_block), ranges = (nblocks + g - 1) / g;
+  const int64_t per_cu = log_block == 15 ? 1 : log_block == 14 ? 2 : 4;  // 1024, 512 or 256 threads
+  const int64_t wgs = device_cus() * per_cu;
+  if (per_cu > 1 && ranges < 2 * wgs) return 1;
+  return ranges > wgs ? (ranges + wgs - 1) / wgs : 1;
+}
+inline int64_t block_bwd_rows(int log_block, int64_t nblocks) {
+  const int64_t per = group_slots_per_wg(log_block) * block_bwd_run(log_block, nblocks);
+  return (nblocks + per - 1) / per;
+}
 // Blocks that one workgroup of the matrix-core backward adds up, and the rows it
 // leaves in `work`: one block per row up to one per CU, beyond that the fewest
 // blocks per row that leave at most one row per CU.
@@ -251,12 +270,13 @@ constexpr int kGroupMaxJobs = 32;
 struct GroupJob {
   const void* src;   // forward: latent [n]; backward: grad of the weight [size] (weight dtype)
   void* dst;         // forward: weight [size] (weight dtype); backward: grad_latent [n]
-  void* part;        // backward: nblocks partial rows of n values, `stride` values apart
+  void* part;        // backward: `rows` partial rows of n values, `stride` values apart
   int64_t size;
   int32_t n;
   int32_t stride;    // 128-byte aligned rows: n rounded up to 32 floats or 64 bfloat16
   int32_t part_bf16; // rows are bfloat16 (the matrix-core chain's backward), else float32
   int32_t nblocks;   // ceil(size / B)
+  int32_t run, rows; // backward: what each workgroup adds up and the rows this leaves, as in the per-module call
   uint32_t seed32;
   int32_t layers;
   int32_t wdtype;    // weight dtype code
@@ -271,11 +291,10 @@ struct GroupTable {
 };
 // Whole-block jobs (B <= 2^15) of one latent dtype, weight dtype and block size
 // (bfht_grouped_kernels.hip).
-int group_slots_per_wg(int log_block);
 hipError_t launch_block_grouped(const GroupTable& g, int dtype, int wdtype, int log_block, hipStream_t s,
                                 bool fwd);
 // bfloat16 jobs of block 2^15 and one layer count on the matrix cores.
-hipError_t launch_mfma15_grouped(const GroupTable& g, int layers, hipStream_t s, bool fwd);
+hipError_t launch_mfma15_grouped(const GroupTable& g, int layers, hipStream_t s, bool fwd, bool summed);
 // Block sums of backward jobs of one latent dtype and one partial-row type
 // (prefix in 256-column tiles).
 constexpr int kGroupReduceCols = 256;

@@ -1,6 +1,6 @@
 // BlockFHT generator kernels at block size 2^15 on the matrix cores: forward
-// (signed bf16 output slice) and backward (float32 per-block partial latent
-// gradients).  The chain itself (layouts, Walsh stages, LDS exchanges, sign
+// (signed bf16 output slice) and backward (bfloat16 partial rows of the latent
+// gradient, one per workgroup).  The chain itself (layouts, Walsh stages, LDS exchanges, sign
 // words) is in bfht_mfma_chain.h.
 //
 // Reference semantics: latent_weight_lab/block_fht.py:84-109 (forward) and
@@ -347,13 +347,9 @@ __device__ __forceinline__ void add_signed(f32x16 (&sum)[kTiles], const f32x16 (
 // 2592 67 / 88 (of which the sum of 2592 rows takes 32); a gradient off the
 // 16-byte grid, read without prefetch, 128 / 134 at 2564 blocks.
 template <int L, bool kWhole>
-__global__ __launch_bounds__(kThreads, 2) void bfht_mfma15_bwd_sum(const __bf16* __restrict__ grad,
-                                                                   __bf16* __restrict__ partial, int n,
-                                                                   int64_t first_block, int64_t nblocks,
-                                                                   int64_t group, int64_t start, int64_t stop,
-                                                                   uint32_t seed32) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(2)];
-  const int64_t b0 = (int64_t)blockIdx.x * group, b1 = b0 + group < nblocks ? b0 + group : nblocks;
+__device__ __forceinline__ void bwd_sum_row(const __bf16* __restrict__ grad, __bf16* __restrict__ row,
+                                            int64_t stride, int64_t first_block, int64_t b0, int64_t b1,
+                                            int64_t start, int64_t stop, uint32_t seed32, unsigned char* lds) {
   f32x16 sum[kTiles] = {};
   u32x4 next[kTiles][2];
   bool loaded = false;  // `next` holds the coming block (a whole, aligned one)
@@ -395,8 +391,20 @@ __global__ __launch_bounds__(kThreads, 2) void bfht_mfma15_bwd_sum(const __bf16*
         v[k][q] = pk(sum[t][r], sum[t][r + 1]);
       }
     }
+  store_row<L, 2>(v, x, lds, row, (uint32_t)stride * 2u);
+}
+
+template <int L, bool kWhole>
+__global__ __launch_bounds__(kThreads, 2) void bfht_mfma15_bwd_sum(const __bf16* __restrict__ grad,
+                                                                   __bf16* __restrict__ partial, int n,
+                                                                   int64_t first_block, int64_t nblocks,
+                                                                   int64_t group, int64_t start, int64_t stop,
+                                                                   uint32_t seed32) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(2)];
+  const int64_t b0 = (int64_t)blockIdx.x * group, b1 = b0 + group < nblocks ? b0 + group : nblocks;
   const int64_t stride = mfma15_part_stride(n);
-  store_row<L, 2>(v, x, lds, partial + (int64_t)blockIdx.x * stride, (uint32_t)stride * 2u);
+  bwd_sum_row<L, kWhole>(grad, partial + (int64_t)blockIdx.x * stride, stride, first_block, b0, b1, start, stop,
+                         seed32, lds);
 }
 
 // ---------------------------------------------------------------- grouped
@@ -438,6 +446,19 @@ __global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_bwd_
   chain_chunks<L, kBufs>(x, lds, src, [](int i) { return L - i; }, v);
   // the row stride is a multiple of 64
   store_row<L, kBufs>(v, x, lds, static_cast<__bf16*>(jb.part) + slot * (int64_t)jb.stride, (uint32_t)jb.stride * 2u);
+}
+
+// The same for jobs of more blocks than CUs, `run` blocks per row.
+template <int L>
+__global__ __launch_bounds__(kThreads, 2) void bfht_mfma15_bwd_sum_grouped(const GroupTable g) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[chain_lds_bytes(2)];
+  const int j = group_job(g, (int)blockIdx.x);
+  const GroupJob& jb = g.job[j];
+  const int64_t index = (int64_t)blockIdx.x - g.prefix[j];
+  const int64_t b0 = index * jb.run, b1 = b0 + jb.run < jb.nblocks ? b0 + jb.run : jb.nblocks;
+  bwd_sum_row<L, false>(static_cast<const __bf16*>(jb.src),
+                        static_cast<__bf16*>(jb.part) + index * (int64_t)jb.stride, jb.stride, 0, b0, b1, 0, jb.size,
+                        jb.seed32, lds);
 }
 
 }  // namespace
@@ -497,7 +518,7 @@ hipError_t launch_mfma15_bwd(const BfhtArgs& a, hipStream_t s) {
 
 }  // namespace
 
-hipError_t launch_mfma15_grouped(const GroupTable& g, int layers, hipStream_t s, bool fwd) {
+hipError_t launch_mfma15_grouped(const GroupTable& g, int layers, hipStream_t s, bool fwd, bool summed) {
   using namespace mfma15;
   if (g.count <= 0 || g.prefix[g.count] == 0) return hipSuccess;
   const dim3 grid((unsigned)g.prefix[g.count]), block(kThreads);
@@ -507,6 +528,8 @@ hipError_t launch_mfma15_grouped(const GroupTable& g, int layers, hipStream_t s,
     hipLaunchKernelGGL((bfht_mfma15_fwd_grouped<L, 1>), grid, block, 0, s, g);              \
   else if (fwd)                                                                             \
     hipLaunchKernelGGL((bfht_mfma15_fwd_grouped<L, 2>), grid, block, 0, s, g);              \
+  else if (summed)                                                                          \
+    hipLaunchKernelGGL((bfht_mfma15_bwd_sum_grouped<L>), grid, block, 0, s, g);             \
   else if (paired)                                                                          \
     hipLaunchKernelGGL((bfht_mfma15_bwd_grouped<L, 1>), grid, block, 0, s, g);              \
   else                                                                                      \

@@ -472,7 +472,7 @@ static_assert(unshuffle_bits(0x55555555u) == 0x0000ffffu && unshuffle_bits(0xaaa
 // layer j, whose stage a runs in S1 (j odd: bit permutation swap_idx34) or S0
 // (j even: swap_idx04); the last one (j = L) is read by the output code, unpermuted.
 // kDirect (the direct-store last layer): slot L - 1 holds the last layer's
-// words as store_direct reads them, unshuffled (unshuffle_bits) and at index
+// words as direct_chunks reads them, unshuffled (unshuffle_bits) and at index
 // (w >> 7) + 8 (w & 127), so that the eight words of a lane's chunks k = w >> 7
 // = 0..7 are consecutive.
 template <int L, bool kDirect = false, class SignLayer>
@@ -529,7 +529,7 @@ __device__ __forceinline__ void read_words(const Ctx& x, const uint32_t* wtab, i
 // its table first (their loads' latency covers the hashing) and read after
 // each layer's exchange barrier, which also orders the table's writes.
 // kDirect (odd L): the last layer ends in layout F (see exchange_slot_final)
-// instead of S1, and `fin` is not read (store_direct reads the last words).
+// instead of S1, and `fin` is not read (direct_chunks reads the last words).
 template <int L, bool kDirect = false, int kBufs = 2, class SignLayer>
 __device__ __forceinline__ void run_chain(f32x16 (&acc)[kTiles], const Ctx& x, unsigned char* lds,
                                           const u32x4 (&src)[kTiles][2], SignLayer sign_layer,

@@ -344,3 +344,24 @@ def test_suspended_cache_keeps_ce_grad_and_live_perturbation_grad(dtype, shape_k
     _check_close(hybrid_perturbed, dynamic_perturbed, dtype)
     _check_close(hybrid.generator.latent.grad, dynamic.generator.latent.grad, dtype)
     _check_close(hybrid.bias.grad, dynamic.bias.grad, dtype)
+
+
+@pytest.mark.parametrize("jobs", [
+    # more than one set of workgroups: several blocks (ranges of blocks) per row, first and last partly filled
+    [(32768, 300 * 32768 - 40, 3, 21, 0.5, BF16, BF16), (30000, 257 * 32768, 2, 22, 1.0, BF16, BF16)],
+    [(30000, 260 * 32768 + 5, 3, 23, 1.0, F32, BF16), (20000, 3 * 32768, 3, 24, 1.0, F32, BF16)],
+    [(8000, 2100 * 8192 - 9, 1, 25, 1.0, F32, F32), (8000, 5 * 8192, 2, 26, 2.0, F32, F32)],
+    [(60, 2_000_000, 2, 27, 1.0, F16, F32), (3000, 5 * 4096 + 1, 3, 28, 1.0, F16, F32)],
+])
+def test_flush_of_large_jobs_matches_per_module_bitwise(jobs):
+    """The flush adds up the same blocks per row as the per-module backward, in the same order."""
+    specs, wants = [], []
+    for i, (n, size, layers, seed, ws, ld, wd) in enumerate(jobs):
+        lat = make_latent(n, ld, 70 + i)
+        gw = torch.randn(size, generator=torch.Generator().manual_seed(170 + i)).to(wd).cuda()
+        specs.append((lat, gw, size, layers, seed, ws, None))
+        wants.append(ws * block_fht_grad_latent(lat, gw.to(ld), size, layers, seed))
+    got = ops.flush_weight_grads(specs)
+    torch.cuda.synchronize()
+    for r, want, job in zip(got, wants, jobs):
+        assert torch.equal(r, want), job
