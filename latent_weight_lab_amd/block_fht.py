@@ -241,7 +241,17 @@ class _BlockFHTLinearFn(torch.autograd.Function):
 
 
 def _generated_weight(latent, size, layers, seed, weight_scale, modulation_alpha):
-    flat = block_fht_slice(latent, int(size), int(layers), int(seed), 0, int(size)) * float(weight_scale)
+    # Without a graph to record (the training linear's own forward and backward) the
+    # grouped weight kernels scale in the generator's stores: the same values as generating
+    # and then multiplying the whole weight once more (5 us of 14 at 768 x 3072).
+    # Generators they do not take go the long way.
+    scaled = None
+    if not (torch.is_grad_enabled() and latent.requires_grad):
+        scaled = ops.materialize_weights([(latent, size, layers, seed, weight_scale, latent.dtype)], strict=False)
+    if scaled is not None:
+        (flat,) = scaled
+    else:
+        flat = block_fht_slice(latent, int(size), int(layers), int(seed), 0, int(size)) * float(weight_scale)
     if float(modulation_alpha) != 0.0:
         flat = flat + float(modulation_alpha) * latent.square().sum()
     return flat

@@ -193,3 +193,29 @@ def test_forward_fused_matches_materialized(opts):
                                           None if lin.bias is None else lin.bias.double())
     assert got.shape == (3, 7, 40)
     assert O.rel_l2(got.double().cpu().numpy(), want.cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("n,size,dtype,strided", [
+    (32768, 70_001, torch.bfloat16, False),   # matrix cores
+    (30000, 70_001, torch.bfloat16, True),    # every second value of a longer latent
+    (3000, 10_007, torch.float16, False),
+    (20000, 70_001, torch.float32, False),
+    (40000, 70_001, torch.float32, False),    # 2^16: generated, then scaled
+])
+def test_training_weight_scaled_in_its_stores_bitwise(n, size, dtype, strided):
+    """The training linear's weight equals the generated one times weight_scale, bit for bit
+    (float16 up to its last bit: the product goes to float16 directly or by way of float32),
+    and still records a graph where one is asked for."""
+    from latent_weight_lab_amd.block_fht import _generated_weight, block_fht_slice
+
+    gen = torch.Generator().manual_seed(n)
+    lat = (torch.randn(2 * n if strided else n, generator=gen) * 0.02).to(dtype).cuda()
+    lat = lat[::2] if strided else lat
+    want = block_fht_slice(lat, size, 3, 17, 0, size) * 0.37
+    got = _generated_weight(lat, size, 3, 17, 0.37, 0.0)
+    if dtype == torch.float16:
+        torch.testing.assert_close(got, want, rtol=2.0 ** -10, atol=2.0 ** -24)
+    else:
+        assert torch.equal(got, want)
+    leaf = lat.detach().requires_grad_(True)
+    assert _generated_weight(leaf, size, 3, 17, 0.37, 0.0).requires_grad
