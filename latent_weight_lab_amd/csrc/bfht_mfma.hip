@@ -13,14 +13,14 @@ namespace mfma15 {
 namespace {
 
 // Runs the chain and leaves this lane's eight signed output chunks in v (odd
-// L: from layout F, even L: from S0), times `scale` after their rounding; chunk k
-// holds block positions chunk_pos<L>(x, k) .. + 7.
-template <int L, int kBufs, class SignLayer>
+// L: from layout F, or from S1 without kDirect; even L: from S0), times `scale` after
+// their rounding; chunk k holds block positions chunk_pos<L, kDirect>(x, k) .. + 7.
+template <int L, int kBufs, bool kDirect = L % 2 == 1, class SignLayer>
 __device__ __forceinline__ void chain_chunks(const Ctx& x, unsigned char* lds, const u32x4 (&src)[kTiles][2],
                                              SignLayer sign_layer, u32x4 (&v)[8], float scale = 1.0f) {
   f32x16 acc[kTiles];
   uint32_t nw[4];
-  if constexpr (L % 2 == 1) {
+  if constexpr (kDirect) {
     run_chain<L, true, kBufs>(acc, x, lds, src, sign_layer, nw);
     direct_chunks(acc, x, reinterpret_cast<const uint32_t*>(lds + kBufs * kXBufBytes) + (L - 1) * kWordsPerLayer, v,
                   scale);
@@ -33,20 +33,20 @@ __device__ __forceinline__ void chain_chunks(const Ctx& x, unsigned char* lds, c
     }
   }
 }
-template <int L>
+template <int L, bool kDirect>
 __device__ __forceinline__ int chunk_pos(const Ctx& x, int k) {
-  return L % 2 == 1 ? direct_chunk_pos(x, k) : out_chunk_pos<L>(x, k);
+  return kDirect ? direct_chunk_pos(x, k) : out_chunk_pos<L>(x, k);
 }
 
 // Puts the chunks into `lds` in position order (chunk c at stage_slot(c)) and
 // waits for every wave's; returns the staged block.
-template <int L, int kBufs>
+template <int L, int kBufs, bool kDirect = L % 2 == 1>
 __device__ __forceinline__ const u32x4* stage_chunks(const u32x4 (&v)[8], const Ctx& x, unsigned char* lds) {
   // two buffers: the one the last layer did not exchange through is free
   u32x4* stage = reinterpret_cast<u32x4*>(lds + (kBufs == 2 ? (L & 1) * kXBufBytes : 0));
   if (kBufs == 1) __syncthreads();  // every wave has read the last exchange
 #pragma unroll
-  for (int k = 0; k < 8; ++k) stage[stage_slot(chunk_pos<L>(x, k) >> 3)] = v[k];
+  for (int k = 0; k < 8; ++k) stage[stage_slot(chunk_pos<L, kDirect>(x, k) >> 3)] = v[k];
   __syncthreads();
   return stage;
 }
@@ -119,19 +119,19 @@ __device__ __forceinline__ void store_range_shifted(const u32x4* stage, __bf16* 
 // launcher checked that) goes out in whole chunks, from registers where they
 // leave the chain 1 KiB contiguous per wave (odd L); a partial block, or an
 // output off that grid, is staged and stored in aligned 16-byte slots.
-template <int L, int kBufs, bool kWhole = false>
+template <int L, int kBufs, bool kWhole = false, bool kDirect = L % 2 == 1>
 __device__ __forceinline__ void store_block(const u32x4 (&v)[8], const Ctx& x, unsigned char* lds, __bf16* oblk,
                                             int lo, int hi) {
   if (kWhole || (lo == 0 && hi == kB && ((uintptr_t)oblk & 15) == 0)) {
     const auto out_r = rsrc(oblk, (uint32_t)(kB * 2));
-    if constexpr (L % 2 == 1)
+    if constexpr (kDirect)
       store_direct(v, x, out_r);
     else
-      store_staged(stage_chunks<L, kBufs>(v, x, lds), out_r);
+      store_staged(stage_chunks<L, kBufs, kDirect>(v, x, lds), out_r);
     return;
   }
   if constexpr (!kWhole) {
-    const u32x4* stage = stage_chunks<L, kBufs>(v, x, lds);
+    const u32x4* stage = stage_chunks<L, kBufs, kDirect>(v, x, lds);
     if ((uintptr_t)oblk & 1) {  // not on the 2-byte grid: element stores
       uint16_t* o16 = reinterpret_cast<uint16_t*>(oblk);
       for (int p = lo + (int)threadIdx.x; p < hi; p += kThreads)
@@ -174,12 +174,22 @@ __global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_mfma15_fwd(
   u32x4 src[kTiles][2];
   load_latent<kWhole>(x, latent, n, src);
   u32x4 v[8];
-  chain_chunks<L, kBufs>(x, lds, src, [](int i) { return i; }, v);
   // block-local output range [lo, hi); out element of block position p is (base - start) + p
   const int64_t base = block * kB;
   const int lo = kWhole ? 0 : (int)(start - base > 0 ? start - base : 0);
   const int hi = kWhole ? kB : (int)(stop - base < kB ? stop - base : kB);
   __bf16* oblk = out + (base - start);
+  // A block that will be staged anyway does without layout F at odd L (a slice of 31
+  // blocks off the 16-byte grid: 7.65 us against 7.92); two chains in one kernel need
+  // more than the 128 registers of workgroups that share a CU.
+  if constexpr (L % 2 == 1 && kBufs == 2 && !kWhole) {
+    if (lo != 0 || hi != kB || ((uintptr_t)oblk & 15) != 0) {
+      chain_chunks<L, kBufs, false>(x, lds, src, [](int i) { return i; }, v);
+      store_block<L, kBufs, false, false>(v, x, lds, oblk, lo, hi);
+      return;
+    }
+  }
+  chain_chunks<L, kBufs>(x, lds, src, [](int i) { return i; }, v);
   store_block<L, kBufs, kWhole>(v, x, lds, oblk, lo, hi);
 }
 
