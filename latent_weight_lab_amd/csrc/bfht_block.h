@@ -435,7 +435,7 @@ struct BwdLds {
 };
 
 template <int LB>
-inline constexpr bool kBwdSingle = Geo<LB>::G == 1 && Geo<LB>::WG < 1024;  // has a kLoop = false variant
+inline constexpr bool kBwdSingle = LB >= 11 && LB <= 14;  // has a kLoop = false variant
 
 // Backward of whole blocks: the adjoint chain D_0 H D_1 ... H D_L on grad scattered
 // into each block, summed over a run of blocks.  A workgroup takes the G blocks
@@ -450,9 +450,9 @@ inline constexpr bool kBwdSingle = Geo<LB>::G == 1 && Geo<LB>::WG < 1024;  // ha
 // latent 2^15, 96 -> 69 us (now bound by the vector unit's butterflies, as the
 // forward is); 2^12, 98 -> 55; 2^10, 231 -> 38; 2^6, 3040 -> 79.  A latent of 1000
 // under 4000 values: one row, so no second launch, 10.2 -> 6.9 us.
-// kLoop = false (2^13 and 2^14, one block per workgroup): no sum, no registers
-// for it (2^14 under 2^22 values took 18.7 us with them, 16.7 without; at 2^15
-// it made no difference).
+// kLoop = false (one range per workgroup, 2^11 .. 2^14): no sum over ranges, no
+// registers for it (2^14 under 2^22 values took 18.7 us with them, 16.7 without;
+// at 2^15 it made no difference).
 template <int LB, class T, bool kLoop, class Load>
 __device__ __forceinline__ void block_bwd_row(Load grad, float* __restrict__ row, T* __restrict__ grad_latent, int n,
                                               int64_t first_block, int64_t index, int run, int64_t start,
@@ -550,7 +550,7 @@ __device__ __forceinline__ void block_bwd_row(Load grad, float* __restrict__ row
       else
         row[p] = s;
     };
-#pragma unroll 1
+#pragma unroll 4
     for (int p = tid & (kCols - 1); p < B; p += kCols) {
       float s = 0.0f;
 #pragma unroll 8
