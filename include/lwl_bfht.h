@@ -301,7 +301,8 @@ int lwl_bfht_check_linear_backward_latent(int dtype, int64_t tokens, int64_t in_
  *                 grad_weight.to(T)), then latent.grad.add_ or assignment)
  *
  * Each block runs the code of the per-module call, so the results are
- * bit-identical to it.  Jobs take latents of length <= 32768 (blocks up to
+ * bit-identical to it (products are rounded to float32 before a 16-bit type; a
+ * float32 flush that accumulates scales and adds in one FMA).  Jobs take latents of length <= 32768 (blocks up to
  * 2^15); bfloat16 latents of block 2^15 need W = bfloat16.  Destinations must
  * not overlap.  Gains, modulation and residual weights stay with the caller.
  * The flush workspace has room for a partial row per block of every job (float32,

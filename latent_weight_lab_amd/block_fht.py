@@ -244,9 +244,10 @@ def _generated_weight(latent, size, layers, seed, weight_scale, modulation_alpha
     # Without a graph to record (the training linear's own forward and backward) the
     # grouped weight kernels scale in the generator's stores: the same values as generating
     # and then multiplying the whole weight once more (5 us of 14 at 768 x 3072).
-    # Generators they do not take go the long way.
+    # Generators they do not take go the long way, and so do float16 latents: torch's
+    # float16 product takes one rounding or two from element to element, the kernels' always two.
     scaled = None
-    if not (torch.is_grad_enabled() and latent.requires_grad):
+    if latent.dtype != torch.float16 and not (torch.is_grad_enabled() and latent.requires_grad):
         scaled = ops.materialize_weights([(latent, size, layers, seed, weight_scale, latent.dtype)], strict=False)
     if scaled is not None:
         (flat,) = scaled
@@ -544,7 +545,8 @@ def prepare_block_fht_weight_cache(model: nn.Module, dtype: torch.dtype | None =
     The generators run together in a few grouped launches (``ops.materialize_weights``);
     a module the grouped kernels do not take (blocks above 2^15, a bfloat16 latent of
     block 2^15 cached in another dtype) materializes on its own.  The cached weights
-    are bit-identical either way.
+    are bit-identical either way, up to the last bit of a float16 product: float32 and
+    then float16 in the grouped kernels, in torch's one rounding for some elements.
     """
     modules = [m for m in model.modules() if isinstance(m, BlockFHTLinear) and _cacheable(m)]
     if not modules or _prepare_plain(modules, dtype):

@@ -62,6 +62,13 @@ template <class T>
 __device__ __forceinline__ T from_f32(float v) {
   return (T)v;
 }
+// v as the float32 it has been computed to: without this the compiler rounds a
+// float32 product straight to float16 when that is where it goes next
+// (v_fma_mixlo_f16), one rounding short of a product followed by a cast.
+__device__ __forceinline__ float as_rounded(float v) {
+  asm("" : "+v"(v));
+  return v;
+}
 
 __device__ __forceinline__ int lds_index(int p) { return p + (p >> 5); }
 

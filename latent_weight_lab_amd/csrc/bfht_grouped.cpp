@@ -11,7 +11,8 @@
 // block — and
 // each class runs in launches of up to kGroupMaxJobs jobs.  Every block runs
 // exactly the code of its per-module launch, so the results are bit-identical
-// to the per-module path followed by torch's scale, cast and accumulate.
+// to the per-module path followed by a scale, cast and accumulate of their own
+// (but that a float32 flush scales and adds in one FMA).
 #include <hip/hip_runtime_api.h>
 
 #include <vector>

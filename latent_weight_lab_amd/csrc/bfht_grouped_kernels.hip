@@ -27,7 +27,7 @@ struct WeightStore {
     buf_store_at<W>(value(v), r, base, c);
   }
   __device__ void at(int64_t i, float v) const { out[i] = from_f32<W>(value(v)); }
-  __device__ float value(float v) const { return round_to<T>(round_to<T>(v) * scale); }
+  __device__ float value(float v) const { return round_to<T>(as_rounded(round_to<T>(v) * scale)); }
 };
 
 // Load: the weight gradient cast to T (torch's `grad.to(latent.dtype)`).

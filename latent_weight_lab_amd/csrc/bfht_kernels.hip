@@ -247,7 +247,9 @@ __global__ __launch_bounds__(256) void bfht_reduce_few(const P* __restrict__ par
 // (the planner rounds the stride up to 32 floats), so loads are 16 bytes wide.
 template <class T>
 __device__ __forceinline__ void grad_store(T* dst, int i, float sum, float scale, int accumulate, float prev) {
-  float r = round_to<T>(round_to<T>(sum) * scale);
+  float r = round_to<T>(sum) * scale;
+  // (float32: the product and the accumulating add are one FMA)
+  if constexpr (sizeof(T) == 2) r = round_to<T>(as_rounded(r));
   if (accumulate) r = prev + r;  // prev: dst[i] as float
   dst[i] = from_f32<T>(r);
 }

@@ -296,8 +296,9 @@ def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = No
     ``block_fht.py:503-563``).
 
     ``specs``: ``(latent, size, layers, seed, weight_scale, weight_dtype)`` per generator.
-    Returns flat weights equal to ``(generate(latent) * weight_scale).to(weight_dtype)``,
-    written into ``outs`` (contiguous, ``size`` elements of ``weight_dtype`` each) when given.
+    Returns flat weights equal to ``(generate(latent) * weight_scale).to(weight_dtype)`` (a
+    float16 product rounded to float32 first), written into ``outs`` (contiguous, ``size``
+    elements of ``weight_dtype`` each) when given.
     ``strict=False``: None instead of an error when the kernels do not take some generator
     (nothing is generated then).
     """
@@ -339,8 +340,9 @@ def flush_weight_grads(specs: list[tuple], strict: bool = True) -> list[torch.Te
     generator; ``into`` is None or a contiguous tensor of the latent's shape and dtype
     that the result is added to in place (``latent.grad.add_``).  Returns, per spec,
     ``into`` or a new tensor holding ``weight_scale * block_fht_grad_latent(latent,
-    grad_weight.to(latent.dtype), ...)``.  ``strict=False``: None instead of an error when
-    the kernels do not take some generator (nothing is added or written then).
+    grad_weight.to(latent.dtype), ...)`` (float32: scaled and added in one FMA).
+    ``strict=False``: None instead of an error when the kernels do not take some generator
+    (nothing is added or written then).
     """
     if not specs:
         return []

@@ -95,6 +95,33 @@ def test_flush_matches_per_module_bitwise():
         assert torch.equal(r, want), JOBS[i]
 
 
+@pytest.mark.parametrize("ld", [F32, F16, BF16])
+@pytest.mark.parametrize("wd", [F32, F16, BF16])
+@pytest.mark.parametrize("n,size", [(10, 231), (700, 5003), (9000, 300_001), (32768, 400_000)])
+def test_roundings_follow_torch_bitwise(n, size, ld, wd):
+    """A scale that is no power of two: the products are rounded to float32 before they go to
+    float16, and a 16-bit result is rounded before it is added.  (So do torch's operators, but
+    for the float16 products its kernels form one element at a time, which it rounds once: the
+    expected values take the steps one by one.)  A float32 product is added in one FMA: half an
+    ulp of the product off the two operators, and the sum's own rounding."""
+    if ld == BF16 and n == 32768 and wd != BF16:
+        pytest.skip("not taken by the grouped kernels")
+    lat = make_latent(n, ld, n)
+    (w,) = ops.materialize_weights([(lat, size, 3, 17, 0.37, wd)])
+    assert torch.equal(w, (ops.forward(lat, size, 3, 17, 0, size).float() * 0.37).to(ld).to(wd))
+    gw = torch.randn(size, generator=torch.Generator().manual_seed(n + 1)).to(wd).cuda()
+    own = (block_fht_grad_latent(lat, gw.to(ld), size, 3, 17).float() * 0.37).to(ld)
+    before = torch.randn(n, generator=torch.Generator().manual_seed(n + 2)).to(ld).cuda()
+    fresh, added = ops.flush_weight_grads([(lat, gw, size, 3, 17, 0.37, None),
+                                           (lat, gw, size, 3, 17, 0.37, before.clone())])
+    assert torch.equal(fresh, own)
+    if ld == F32:
+        off = (added - (before + own)).abs()
+        assert (off <= own.abs() * 2.0 ** -24 + (before + own).abs() * 2.0 ** -23).all()
+    else:
+        assert torch.equal(added, (before.float() + own.float()).to(ld))
+
+
 @pytest.mark.parametrize("ld,tol", [(F32, 1e-5), (BF16, 1e-2)])
 def test_flush_matches_oracle(ld, tol):
     n, size, layers, seed, ws = 30000, 200 * 700, 2, 23, 2.0
