@@ -49,15 +49,18 @@ struct LdsWeightStore {
 constexpr int kQuad = 4;  // tokens per team pass
 constexpr int kSpan = 8;  // k iterations of a lane whose x loads are in flight together
 
-// LDS of a workgroup: the generator's exchange buffers and sign tables, then
-// (over them, once they are read) the weight tile and the staged x of one token
-// quad.  4096 staged values keep a 2^14 block at 80 KiB, so that two workgroups
-// share a CU (grouped launches); kWide holds as many as the generator's LDS.
+// LDS of a workgroup.  Narrow: the generator's exchange buffers and sign tables,
+// then (over them, once they are read) the weight tile and the staged x of one
+// token quad, 4096 values of it, so that a 2^14 block takes 80 KiB and two
+// workgroups share a CU.  Wide: the weight tile behind the generator's LDS, which
+// holds a single token's staged x afterwards; one workgroup per CU at 2^14, two below.
 template <int LB, bool kWide>
 struct SmallLinearGeo {
   using Gm = Geo<LB>;
   static constexpr int kTileElems = Gm::G * Gm::B;  // weights generated per workgroup
   static constexpr int kStage = kWide ? BlockLds<LB>::FLOATS : 4096;
+  static constexpr int kTile = kWide ? BlockLds<LB>::FLOATS : 0;   // where the weight tile starts
+  static constexpr int kStaged = kWide ? 0 : kTileElems;           // and the staged x
   static constexpr int kNeed = kTileElems + kStage;
   static constexpr int kLdsFloats = kNeed > BlockLds<LB>::FLOATS ? kNeed : BlockLds<LB>::FLOATS;
   static_assert(kLdsFloats * 4 <= 160 * 1024 && (kWide || LB > 14 || kLdsFloats * 8 <= 160 * 1024), "LDS of one CU");
@@ -72,7 +75,7 @@ __device__ __forceinline__ void small_item(const T* __restrict__ x, const T* __r
                                            int split, const LinearEpi& ep, float* smem) {
   using Gm = Geo<LB>;
   using SG = SmallLinearGeo<LB, kWide>;
-  float* wt = smem;  // the weight tile, row-major [rows][in]
+  float* wt = smem + SG::kTile;  // the weight tile, row-major [rows][in]
   const int64_t size = (int64_t)in_f * out_f;
   const int64_t base = tile * SG::kTileElems;
 
@@ -83,7 +86,7 @@ __device__ __forceinline__ void small_item(const T* __restrict__ x, const T* __r
   const int q1 = q0 + per_split < quads ? q0 + per_split : quads;
   const auto x_r = tile_rsrc(x, (uint64_t)tokens * in_f * sizeof(T));
   const int nstage = (int)small_stage(tokens, in_f);
-  const bool staged = nstage <= SG::kStage;
+  const bool staged = kWide ? tokens == 1 : nstage <= SG::kStage;
   // thread's share i0 + e * WG (e < kSpan) of quad q's staged x (tokens past the batch read 0)
   auto stage_load = [&](int q, int i0, float (&v)[kSpan]) {
 #pragma unroll
@@ -102,7 +105,7 @@ __device__ __forceinline__ void small_item(const T* __restrict__ x, const T* __r
   // 1. the tile's G blocks (inactive slots past the last block store nothing;
   //    their rows lie past out_features and are never read)
   const int64_t slot = tile * Gm::G + (threadIdx.x >> Gm::LT);
-  block_fwd_slot<LB, T, Gm::G, true>(latent, LdsWeightStore{wt, base, scale}, n, 0, slot, nblocks, 0, size, seed32,
+  block_fwd_slot<LB, T, Gm::G, !kWide>(latent, LdsWeightStore{wt, base, scale}, n, 0, slot, nblocks, 0, size, seed32,
                                      layers, smem);
   __syncthreads();
 
@@ -223,11 +226,11 @@ __device__ __forceinline__ void small_item(const T* __restrict__ x, const T* __r
   using Two = std::integral_constant<int, 2>;
   using Quad = std::integral_constant<int, kQuad>;
   if (staged) {
-    // Each quad's x rows are staged once behind the weight tile and every team
-    // reads them there: read from memory, all the workgroup's passes (and all
-    // the workgroups of an XCD, at decode batches) ask its L2 for the same
-    // few lines.  Tokens past the batch stage as 0.
-    float* xs = smem + SG::kTileElems;
+    // Each quad's x rows are staged once and every team reads them there: read
+    // from memory, all the workgroup's passes (and all the workgroups of an XCD,
+    // at decode batches) ask its L2 for the same few lines.  Tokens past the
+    // batch stage as 0.
+    float* xs = smem + SG::kStaged;
     for (int q = q0; q < q1; ++q) {
       if (q > q0) __syncthreads();  // every team has read the previous quad
       for (int i0 = (int)threadIdx.x; i0 < nstage; i0 += kSpan * Gm::WG) {
@@ -326,9 +329,24 @@ hipError_t launch_small_lb(const LinearArgs& a, hipStream_t s) {
   using Gm = Geo<LB>;
   const int64_t wtiles = (a.nblocks_w + Gm::G - 1) / Gm::G;
   const int log_in = log2_of(a.in_features);
-  // x of a quad that needs more than the narrow form's staging but fits the wide one's
+  // The narrow form wherever it stages a quad's x.  A longer row is staged alone (one
+  // token, wide: 16384 -> 1000 in float32 107 -> 65 us) or read by every team from the
+  // caches (several tokens): with a quad staged in rounds its loads were waited out
+  // between barriers (4096 -> 1000, 1000 tokens: float32 1981 -> 715 us, float16 2034 ->
+  // 772).  Of those calls the wide form takes the ones that fit one workgroup per CU,
+  // which gain nothing from the second (16384 -> 64, 16 tokens: 30.4 against 33.9 us; 8192
+  // -> 1000, 15 tokens, 500 workgroups: 47 against 37), and float32 calls whose x no longer
+  // stays in the last-level cache while many rounds of workgroups stream it: twice as
+  // many drift twice as far apart (16384 -> 4096: 512 tokens, 32 MiB, 7.3 against 5.6 ms;
+  // 1000 tokens 14.1 against 24.7; 4003 tokens 57 against 125.  4096 -> 10000: 4003 tokens
+  // 36 against 29; 8000 tokens 72 against 85.  The line keeps every measured call from losing, at the
+  // price of a few that would still gain).  float16 keeps its lead to 2^29 bytes of x.
   const int64_t nstage = small_stage(a.tokens, a.in_features);
-  const bool wide = LB > 10 && nstage > SmallLinearGeo<LB, false>::kStage && nstage <= SmallLinearGeo<LB, true>::kStage;
+  const bool one_per_cu = wtiles * a.token_splits <= device_cus();
+  const bool streams_x = sizeof(T) == 4 && a.tokens * a.in_features * 4 >= ((int64_t)48 << 20) &&
+                         (double)(a.tokens * a.in_features) * (double)(a.in_features * a.out_features) >= 5e14;
+  const bool wide =
+      LB > 10 && nstage > SmallLinearGeo<LB, false>::kStage && (a.tokens == 1 || one_per_cu || streams_x);
 #define LWL_SMALL(W)                                                                                                \
   hipLaunchKernelGGL((bfht_linear_small<LB, T, W>), dim3((unsigned)wtiles, (unsigned)a.token_splits), dim3(Gm::WG), \
                      0, s, (const T*)a.x, (const T*)a.latent, (T*)a.out, (int)a.tokens, (int)a.in_features, log_in, \

@@ -235,3 +235,28 @@ def test_small_domain_gradients_match_generated_route():
         grads.append((y.detach(), la.grad, xa.grad))
     for a, b in zip(*grads):
         assert O.rel_l2(a.double().cpu().numpy(), b.double().cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("in_f,out_f,n", [
+    (16384, 300, 16384),   # one row per block, 300 workgroups: more than one per CU from the start
+    (16384, 40, 9000),     # 40 workgroups, one per CU up to 6 token ranges
+    (8192, 130, 8000),     # block 2^13
+    (4096, 70, 4000),      # block 2^12, two blocks per workgroup
+    (2048, 60, 2048),      # block 2^11: four
+])
+def test_long_rows_one_result_whatever_the_form(in_f, out_f, n, dtype):
+    """Rows too long for a quad's x to be staged: a single token is staged alone, several are
+    read from memory, with one workgroup per CU or with two.  Every form adds a row's products
+    in the same order, so a token's outputs do not depend on its batch."""
+    g = torch.Generator().manual_seed(in_f + out_f)
+    latent = (torch.randn(n, generator=g) * 0.1).to(dtype).cuda()
+    # (16 rows of 2048 per 16-bit tile: from 16 tokens the matrix-core variant's, another order)
+    most = 15 if in_f == 2048 and dtype != torch.float32 else 1025
+    x = torch.randn(most, in_f, generator=g).to(dtype).cuda()
+    whole = ops.linear_forward(x, latent, out_f, 2, 5, 0.5)
+    rel = O.rel_l2(whole[:130].double().cpu().numpy(), oracle_out(x[:130], latent, out_f, 2, 5, 0.5))
+    assert rel < TOL[dtype]
+    for tokens in (1, 2, 4, 7, 14, 128, 129, 700):
+        if tokens <= most:
+            assert torch.equal(ops.linear_forward(x[:tokens], latent, out_f, 2, 5, 0.5), whole[:tokens]), tokens
