@@ -246,11 +246,9 @@ def _generated_weight(latent, size, layers, seed, weight_scale, modulation_alpha
     # and then multiplying the whole weight once more (5 us of 14 at 768 x 3072).
     # Generators they do not take go the long way, and so do float16 latents: torch's
     # float16 product takes one rounding or two from element to element, the kernels' always two.
-    scaled = None
-    if latent.dtype != torch.float16 and not (torch.is_grad_enabled() and latent.requires_grad):
-        scaled = ops.materialize_weights([(latent, size, layers, seed, weight_scale, latent.dtype)], strict=False)
-    if scaled is not None:
-        (flat,) = scaled
+    if (latent.dtype != torch.float16 and ops.weight_job_taken(latent, int(size), latent.dtype)
+            and not (torch.is_grad_enabled() and latent.requires_grad)):
+        (flat,) = ops.materialize_weights([(latent, size, layers, seed, weight_scale, latent.dtype)])
     else:
         flat = block_fht_slice(latent, int(size), int(layers), int(seed), 0, int(size)) * float(weight_scale)
     if float(modulation_alpha) != 0.0:
@@ -511,8 +509,9 @@ def forward_fused_grouped(modules: list["BlockFHTLinear"], inputs: list[torch.Te
     ``forward_fused`` would run as one fused launch: at decode batch sizes one matrix fills
     a fraction of the chip, and the grouped launch runs all of them together (not in the
     reference, which calls ``ext.linear_forward`` per matrix, ``block_fht.py:274``).  Each
-    job carries its module's epilogue (bias in the grouped kernels; modulation or residual
-    base make it a single launch inside the call).  Outputs equal the per-module calls bit
+    job carries its module's epilogue (bias, and in the reference's domain a residual base,
+    in the grouped kernels; modulation, or a base elsewhere, makes it a single launch inside
+    the call).  Outputs equal the per-module calls bit
     for bit.  Other modules, and calls that record gradients, run ``forward_fused`` one
     by one."""
     if len(modules) != len(inputs):
@@ -548,60 +547,45 @@ def prepare_block_fht_weight_cache(model: nn.Module, dtype: torch.dtype | None =
     are bit-identical either way, up to the last bit of a float16 product: float32 and
     then float16 in the grouped kernels, in torch's one rounding for some elements.
     """
-    modules = [m for m in model.modules() if isinstance(m, BlockFHTLinear) and _cacheable(m)]
-    if not modules or _prepare_plain(modules, dtype):
-        return
-    grouped, specs = [], []
-    for module in modules:
+    # A training step's prepare and flush are host-bound (24 matrices: 190 us of kernels):
+    # jobs are chosen by block size and dtypes, so that only what the kernels take is
+    # allocated and packed, the library checks all of them in the one call, and plain
+    # weights are made in their final shape (24 float32 latents, bfloat16 weights, prepare
+    # and flush together: 515 us with a library check and views per module, 350 so).
+    grouped, specs, outs = [], [], []
+    for module in model.modules():
+        if not isinstance(module, BlockFHTLinear) or not _cacheable(module):
+            continue
         g = module.generator
-        latent = g.latent
+        latent, size = g.latent, g.size
         plain = not module._cache_needs_torch_epilogue()
         # the kernel's output dtype: the cache dtype when it finishes the weight
         wdtype = (dtype or latent.dtype) if plain else latent.dtype
-        if ops.weight_job_supported(latent, g.size, g.layers, wdtype):
-            grouped.append((module, plain))
-            specs.append((latent, g.size, g.layers, g.seed, module.weight_scale, wdtype))
-        else:
+        if not (latent.is_cuda and latent.is_contiguous() and ops.weight_job_taken(latent, size, wdtype)):
             module.materialize_weight_cache(dtype=dtype)
+            continue
+        out_f, in_f = module.out_features, module.in_features
+        done = plain and size == out_f * in_f
+        grouped.append((module, done))
+        specs.append((latent, size, g.layers, g.seed, module.weight_scale, wdtype))
+        outs.append(torch.empty((out_f, in_f) if done else (size,), dtype=wdtype, device=latent.device))
     if not specs:
         return
-    with torch.no_grad():
-        weights = ops.materialize_weights(specs)
-        for (module, plain), w in zip(grouped, weights):
-            if not plain:
-                w = module._finish_weight(w)
-                if dtype is not None:
-                    w = w.to(dtype=dtype)
-            module._cached_weight = w.view(module.out_features, module.in_features).detach().requires_grad_(True)
-
-
-def _cache_latent(latent: torch.Tensor) -> bool:
-    # the tensor-side half of ops.weight_job_supported (the library checks the rest)
-    return latent.is_cuda and latent.is_contiguous() and latent.dtype in _native.DTYPE_CODES
-
-
-def _prepare_plain(modules, dtype) -> bool:
-    """Every cache in one call, without asking the library about each module first: all of
-    ``modules`` plain and taken by the grouped kernels (else False, nothing done).  A training
-    step's prepare and flush are host-bound (24 matrices: 190 us of kernels); with one library
-    call per direction, jobs packed by struct and no views they take 350 us instead of 515."""
-    if dtype is not None and dtype not in _native.DTYPE_CODES:
-        return False
-    specs, outs = [], []
-    for module in modules:
-        g = module.generator
-        latent = g.latent
-        if (module._cache_needs_torch_epilogue() or not _cache_latent(latent)
-                or g.size != module.in_features * module.out_features):
-            return False
-        wdtype = dtype or latent.dtype
-        specs.append((latent, g.size, g.layers, g.seed, module.weight_scale, wdtype))
-        outs.append(torch.empty((module.out_features, module.in_features), dtype=wdtype, device=latent.device))
-    if ops.materialize_weights(specs, outs, strict=False) is None:
-        return False
-    for module, w in zip(modules, outs):
+    ops.materialize_weights(specs, outs)
+    for (module, done), w in zip(grouped, outs):
+        if not done:
+            w = _finished(module, w, dtype)
         module._cached_weight = w.requires_grad_(True)
-    return True
+
+
+@torch.no_grad()
+def _finished(module: "BlockFHTLinear", w: torch.Tensor, dtype: torch.dtype | None) -> torch.Tensor:
+    # a generated weight of a module with options applied in torch, as its own call finishes it
+    if module._cache_needs_torch_epilogue():
+        w = module._finish_weight(w)
+        if dtype is not None:
+            w = w.to(dtype=dtype)
+    return w.view(module.out_features, module.in_features).detach()
 
 
 def flush_block_fht_weight_cache(model: nn.Module) -> None:
@@ -612,81 +596,44 @@ def flush_block_fht_weight_cache(model: nn.Module) -> None:
     which also scale by weight_scale and add into ``latent.grad``; gains and
     modulation are applied in torch around them, as in the per-module flush.
     """
-    live = []
+    grouped, specs, targets = [], [], set()
     for module in model.modules():
         if not isinstance(module, BlockFHTLinear) or module._cached_weight is None:
             continue
-        if module._cached_weight.grad is None:
+        source = module._cached_weight.grad
+        if source is None:
             module._cached_weight = None
-        else:
-            live.append(module)
-    if not live or _flush_plain(live):
-        return
-    grouped, specs, targets = [], [], set()
-    for module in live:
-        cached = module._cached_weight
+            continue
         g = module.generator
         latent = g.latent
         plain = not module._cache_needs_torch_epilogue()
-        if plain:
-            source = cached.grad.contiguous().reshape(-1)
-            supported = ops.weight_job_supported(latent, g.size, g.layers, source.dtype, source)
-        else:
-            # the source is the generated-weight gradient in the latent dtype
-            supported = ops.weight_job_supported(latent, g.size, g.layers, latent.dtype)
-        if not supported:
+        # (not plain: the source is the generated-weight gradient in the latent dtype)
+        if not (latent.is_cuda and latent.is_contiguous() and source.is_cuda
+                and (ops.weight_job_taken(latent, g.size, source.dtype, source) if plain
+                     else ops.weight_job_taken(latent, g.size, latent.dtype))):
             module.flush_weight_cache_to_latent_grad()
             continue
         if not plain:
             source = module._generated_weight_grad()
-        into = None
-        if (plain and latent.grad is not None and latent.grad.is_contiguous() and latent.grad.dtype == latent.dtype
-                and id(latent) not in targets):
-            into = latent.grad  # the kernel adds in place (a latent shared by modules: the first only)
+        into = latent.grad
+        if into is not None and not (plain and into.is_contiguous() and into.dtype == latent.dtype
+                                     and id(latent) not in targets):
+            into = None  # else the kernel adds in place (a latent shared by modules: the first only)
         targets.add(id(latent))
-        grouped.append((module, plain, source, into))
+        grouped.append((module, plain, latent, source, into))
         specs.append((latent, source, g.size, g.layers, g.seed, module.weight_scale, into))
     if not specs:
         return
-    with torch.no_grad():
-        results = ops.flush_weight_grads(specs)
-    for (module, plain, source, into), r in zip(grouped, results):
-        latent = module.generator.latent
-        if into is not None:
-            pass  # added in place
-        elif plain:
-            if latent.grad is None:
+    results = ops.flush_weight_grads(specs)
+    for (module, plain, latent, source, into), r in zip(grouped, results):
+        if into is None:  # else added in place
+            if not plain:
+                module._add_latent_grad(r, source)
+            elif latent.grad is None:
                 latent.grad = r
             else:
                 latent.grad.add_(r)
-        else:
-            module._add_latent_grad(r, source)
         module._cached_weight = None
-
-
-def _flush_plain(modules) -> bool:
-    """Every flush in one call, without asking the library about each module first: all of
-    ``modules`` plain, with a latent of their own, and taken by the grouped kernels (else
-    False, nothing done)."""
-    specs, seen = [], set()
-    for module in modules:
-        g = module.generator
-        latent = g.latent
-        source, into = module._cached_weight.grad, latent.grad
-        if (module._cache_needs_torch_epilogue() or not _cache_latent(latent) or id(latent) in seen
-                or not source.is_cuda or source.dtype not in _native.DTYPE_CODES
-                or (into is not None and not (into.is_contiguous() and into.dtype == latent.dtype))):
-            return False
-        seen.add(id(latent))
-        specs.append((latent, source, g.size, g.layers, g.seed, module.weight_scale, into))
-    results = ops.flush_weight_grads(specs, strict=False)
-    if results is None:
-        return False
-    for module, spec, r in zip(modules, specs, results):
-        if spec[6] is None:
-            spec[0].grad = r
-        module._cached_weight = None
-    return True
 
 
 def suspend_block_fht_weight_cache(model: nn.Module) -> list[tuple[BlockFHTLinear, torch.Tensor]]:

@@ -263,9 +263,21 @@ def _pack_job(arr: ctypes.Array, i: int, latent: torch.Tensor, size: int, layers
                    accumulate)
 
 
-def _refused(rc: int) -> bool:
-    """A job the grouped kernels do not take (nothing was launched)."""
-    return rc in (N.LWL_ERR_INVALID, N.LWL_ERR_UNSUPPORTED)
+# (latent dtype, weight dtype) -> the longest latent that the grouped weight kernels take whatever
+# its pointers: blocks of up to 2^15; bfloat16 blocks of 2^15 (the matrix cores) have bfloat16 weights
+_JOB_LATENT = {(d, w): 16384 if d == torch.bfloat16 != w else 32768 for d in N.DTYPE_CODES for w in N.DTYPE_CODES}
+
+
+def weight_job_taken(latent: torch.Tensor, size: int, weight_dtype: torch.dtype,
+                     grad_weight: torch.Tensor | None = None) -> bool:
+    """Whether the grouped weight kernels take this generator by its block, size and dtypes
+    (``lwl_bfht_check_weight_jobs``'s rule without a call of the library: half a us of host
+    time instead of 7), so that nothing is allocated or packed for one they do not take."""
+    n, most = latent.numel(), _JOB_LATENT.get((latent.dtype, weight_dtype), 0)
+    if n <= most:
+        # at most 2^31 - 1 blocks
+        return size <= 0x7FFFFFFF or (size - 1) >> (n - 1).bit_length() < 0x7FFFFFFF
+    return 0 < most < n <= 32768 and weight_job_supported(latent, size, 1, weight_dtype, grad_weight)
 
 
 def weight_job_supported(latent: torch.Tensor, size: int, layers: int, weight_dtype: torch.dtype,
@@ -289,8 +301,7 @@ def weight_job_supported(latent: torch.Tensor, size: int, layers: int, weight_dt
     return N.lib().lwl_bfht_check_weight_jobs(arr, 1, int(grad_weight is None)) == N.LWL_OK
 
 
-def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = None,
-                        strict: bool = True) -> list[torch.Tensor] | None:
+def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = None) -> list[torch.Tensor]:
     """Generate whole weights of many generators in a few launches (the per-module
     ``materialize_weight_cache`` calls of the reference's ``prepare_block_fht_weight_cache``,
     ``block_fht.py:503-563``).
@@ -299,8 +310,6 @@ def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = No
     Returns flat weights equal to ``(generate(latent) * weight_scale).to(weight_dtype)`` (a
     float16 product rounded to float32 first), written into ``outs`` (contiguous, ``size``
     elements of ``weight_dtype`` each) when given.
-    ``strict=False``: None instead of an error when the kernels do not take some generator
-    (nothing is generated then).
     """
     if not specs:
         return []
@@ -324,14 +333,11 @@ def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = No
         result.append(out)
     L = N.lib()
     with _device_guard(dev):
-        rc = L.lwl_bfht_materialize_weights(arr, len(specs), N.stream_ptr(dev))
-    if not strict and _refused(rc):
-        return None
-    N.check(rc)
+        N.check(L.lwl_bfht_materialize_weights(arr, len(specs), N.stream_ptr(dev)))
     return result
 
 
-def flush_weight_grads(specs: list[tuple], strict: bool = True) -> list[torch.Tensor] | None:
+def flush_weight_grads(specs: list[tuple]) -> list[torch.Tensor]:
     """Project many weight gradients back onto their latents in a few launches (the
     per-module ``flush_weight_cache_to_latent_grad`` calls of the reference's
     ``flush_block_fht_weight_cache``, ``block_fht.py:514-569``).
@@ -341,8 +347,6 @@ def flush_weight_grads(specs: list[tuple], strict: bool = True) -> list[torch.Te
     that the result is added to in place (``latent.grad.add_``).  Returns, per spec,
     ``into`` or a new tensor holding ``weight_scale * block_fht_grad_latent(latent,
     grad_weight.to(latent.dtype), ...)`` (float32: scaled and added in one FMA).
-    ``strict=False``: None instead of an error when the kernels do not take some generator
-    (nothing is added or written then).
     """
     if not specs:
         return []
@@ -367,11 +371,8 @@ def flush_weight_grads(specs: list[tuple], strict: bool = True) -> list[torch.Te
     L = N.lib()
     with _device_guard(dev):
         ws_ptr, ws_size, ws = N.workspace(L.lwl_bfht_flush_weight_grads_workspace_size(arr, len(specs)), dev)
-        rc = L.lwl_bfht_flush_weight_grads(arr, len(specs), ws_ptr, ws_size, N.stream_ptr(dev))
+        N.check(L.lwl_bfht_flush_weight_grads(arr, len(specs), ws_ptr, ws_size, N.stream_ptr(dev)))
     del ws, keep
-    if not strict and _refused(rc):
-        return None
-    N.check(rc)
     return outs
 
 

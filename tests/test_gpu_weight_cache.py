@@ -392,3 +392,35 @@ def test_flush_of_large_jobs_matches_per_module_bitwise(jobs):
     torch.cuda.synchronize()
     for r, want, job in zip(got, wants, jobs):
         assert torch.equal(r, want), job
+
+
+@pytest.mark.parametrize("ld,cache_dtype,n", [(F32, BF16, 40000), (BF16, F32, 32768), (BF16, None, 33000)])
+def test_only_what_the_grouped_kernels_take_is_packed(monkeypatch, ld, cache_dtype, n):
+    """A module the grouped kernels do not take costs the others nothing: no job is packed for
+    it and refused, in a prepare and flush or in a training linear, and each of the others is
+    packed once per call.  The results are the per-module calls'."""
+    torch.manual_seed(1)
+    a = torch.nn.ModuleList([BlockFHTLinear(64, 96, bias=False, latent_dim=500, layers=2, seed=1),
+                             BlockFHTLinear(256, 300, bias=False, latent_dim=n, layers=2, seed=2),
+                             BlockFHTLinear(96, 64, bias=False, latent_dim=3000, layers=3, seed=3)]).cuda().to(ld)
+    b = copy.deepcopy(a)
+    packed, pack = [], ops._pack_job
+    monkeypatch.setattr(ops, "_pack_job", lambda arr, i, latent, *args, **kw: (
+        packed.append(latent.numel()) if len(arr) > 1 or latent.numel() < n else None,
+        pack(arr, i, latent, *args, **kw))[1])
+    prepare_block_fht_weight_cache(a, dtype=cache_dtype)
+    per_module_prepare(b, cache_dtype)
+    for ma, mb in zip(a, b):
+        assert torch.equal(ma._cached_weight, mb._cached_weight)
+        ma._cached_weight.grad = torch.randn_like(ma._cached_weight)
+        mb._cached_weight.grad = ma._cached_weight.grad.clone()
+    flush_block_fht_weight_cache(a)
+    assert packed == [500, 3000, 500, 3000]
+    per_module_flush(b)
+    for ma, mb in zip(a, b):
+        assert torch.equal(ma.generator.latent.grad, mb.generator.latent.grad)
+    if n > 32768:  # a training linear with such a latent
+        packed.clear()
+        monkeypatch.setattr(ops, "_pack_job", lambda *args, **kw: packed.append(args) or pack(*args, **kw))
+        a[1](torch.randn(4, 256, device="cuda", dtype=ld)).sum().backward()
+        assert not packed
