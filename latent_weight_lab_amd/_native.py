@@ -196,14 +196,14 @@ def workspace(nbytes: int, device: torch.device) -> tuple[int, int, torch.Tensor
 
 
 def require_cuda(*tensors: torch.Tensor) -> torch.device:
-    dev = None
+    dev = index = None
     for t in tensors:
         if not t.is_cuda:
             raise RuntimeError(
                 "latent_weight_lab_amd runs BlockFHT on the GPU only; move the latent and inputs "
                 "to a cuda device (this package has no CPU path)")
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise RuntimeError(f"latent_weight_lab_amd: tensors on different devices ({dev}, {t.device})")
     return dev

@@ -552,7 +552,7 @@ def prepare_block_fht_weight_cache(model: nn.Module, dtype: torch.dtype | None =
     # allocated and packed, the library checks all of them in the one call, and plain
     # weights are made in their final shape (24 float32 latents, bfloat16 weights, prepare
     # and flush together: 515 us with a library check and views per module, 350 so).
-    grouped, specs, outs = [], [], []
+    grouped, specs, shapes = [], [], []
     for module in model.modules():
         if not isinstance(module, BlockFHTLinear) or not _cacheable(module):
             continue
@@ -568,11 +568,10 @@ def prepare_block_fht_weight_cache(model: nn.Module, dtype: torch.dtype | None =
         done = plain and size == out_f * in_f
         grouped.append((module, done))
         specs.append((latent, size, g.layers, g.seed, module.weight_scale, wdtype))
-        outs.append(torch.empty((out_f, in_f) if done else (size,), dtype=wdtype, device=latent.device))
+        shapes.append((out_f, in_f) if done else (size,))
     if not specs:
         return
-    ops.materialize_weights(specs, outs)
-    for (module, done), w in zip(grouped, outs):
+    for (module, done), w in zip(grouped, ops.materialize_weights(specs, shapes=shapes)):
         if not done:
             w = _finished(module, w, dtype)
         module._cached_weight = w.requires_grad_(True)

@@ -258,9 +258,11 @@ def _pack_job(arr: ctypes.Array, i: int, latent: torch.Tensor, size: int, layers
               weight_dtype: torch.dtype, weight: int = 0, grad_weight: int = 0, grad_latent: int = 0,
               accumulate: int = 0) -> None:
     seed = (int(seed) + (1 << 63)) % (1 << 64) - (1 << 63)  # the int64 with the same low 64 bits
+    dtype, codes = latent.dtype, N.DTYPE_CODES
+    if dtype not in codes or weight_dtype not in codes:
+        N.dtype_code(dtype), N.dtype_code(weight_dtype)  # one of them raises
     _JOB.pack_into(arr, i * _JOB_BYTES, latent.data_ptr(), weight, grad_weight, grad_latent, latent.numel(), int(size),
-                   int(layers), seed, N.dtype_code(latent.dtype), N.dtype_code(weight_dtype), float(weight_scale),
-                   accumulate)
+                   int(layers), seed, codes[dtype], codes[weight_dtype], float(weight_scale), accumulate)
 
 
 # (latent dtype, weight dtype) -> the longest latent that the grouped weight kernels take whatever
@@ -301,7 +303,8 @@ def weight_job_supported(latent: torch.Tensor, size: int, layers: int, weight_dt
     return N.lib().lwl_bfht_check_weight_jobs(arr, 1, int(grad_weight is None)) == N.LWL_OK
 
 
-def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = None) -> list[torch.Tensor]:
+def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = None,
+                        shapes: list[tuple[int, ...]] | None = None) -> list[torch.Tensor]:
     """Generate whole weights of many generators in a few launches (the per-module
     ``materialize_weight_cache`` calls of the reference's ``prepare_block_fht_weight_cache``,
     ``block_fht.py:503-563``).
@@ -309,7 +312,7 @@ def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = No
     ``specs``: ``(latent, size, layers, seed, weight_scale, weight_dtype)`` per generator.
     Returns flat weights equal to ``(generate(latent) * weight_scale).to(weight_dtype)`` (a
     float16 product rounded to float32 first), written into ``outs`` (contiguous, ``size``
-    elements of ``weight_dtype`` each) when given.
+    elements of ``weight_dtype`` each) when given, or made in ``shapes`` (``size`` elements each).
     """
     if not specs:
         return []
@@ -323,7 +326,9 @@ def materialize_weights(specs: list[tuple], outs: list[torch.Tensor] | None = No
             latent = latent.detach().contiguous()
             keep.append(latent)
         if outs is None:
-            out = torch.empty(int(size), dtype=weight_dtype, device=dev)
+            out = torch.empty(int(size) if shapes is None else shapes[i], dtype=weight_dtype, device=dev)
+            if out.numel() != size:
+                raise N.BlockFHTArgumentError(f"shape {i}, {tuple(out.shape)}, must hold {size} elements")
         else:
             out = outs[i]
             if (out.dtype != weight_dtype or out.numel() != int(size) or not out.is_contiguous()
