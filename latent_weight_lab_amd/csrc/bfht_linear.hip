@@ -760,8 +760,8 @@ __global__ __launch_bounds__(256) void bfht_linear_combine(const float* __restri
 // barrier or two each, the scatter, one short contraction on few waves), so with
 // more blocks than CUs two workgroups share each CU (kBufs = 1): half the LDS
 // each, at most 128 VGPRs, one workgroup's waits filled by the other (the 48
-// matrices of a 12-layer GPT-2-small stack, combine included: 134-139 -> 98-100 us
-// at one token, 173 -> 131 at 64, 320 -> 296 at 200; 8 matrices 28.9 -> 25.3).
+// matrices of a 12-layer GPT-2-small stack, combine included: 132 -> 86 us at 8
+// tokens, 172 -> 118 at 64, 317 -> 253 at 200; 8 matrices 28 -> 20 at 8).
 template <int L, int NT, bool kBias, int kBufs>
 __global__ __launch_bounds__(kThreads, kBufs == 1 ? 4 : 2) void bfht_linear_mfma15_grouped(const LinearGroupTable g) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[kBufs == 1 ? kSharedCuLdsBytes : kLinearLdsBytes];
@@ -921,6 +921,16 @@ hipError_t launch_group_chunk(const LinearArgs* const* jobs, int count, int nt, 
   if (split > min_tiles) split = min_tiles;
   if (split < 1) split = 1;
   share_cu = share_cu && chains_share_cu(total * split);
+  // Blocks of long rows contract longest (k steps x token tiles).  First in the grid they
+  // spread over the CUs and the others join them; where two such workgroups met on a CU
+  // while others stood idle, the 8 matrices of two GPT-2-small blocks (432 workgroups) took
+  // 86 us at 200 tokens (one workgroup per CU 66, this order 59), those of four 121 (123, 101).
+  std::vector<const LinearArgs*> order(jobs, jobs + count);
+  if (share_cu)
+    std::stable_sort(order.begin(), order.end(), [](const LinearArgs* a, const LinearArgs* b) {
+      auto cost = [](const LinearArgs* j) { return linear_steps(j->in_features) * ((j->tokens + kTokTile - 1) / kTokTile); };
+      return cost(a) > cost(b);
+    });
   // partial rows: offsets from the lowest `work` (every job's lies in one
   // 256-byte-aligned workspace)
   g.partial = (float*)jobs[0]->work;
@@ -928,7 +938,7 @@ hipError_t launch_group_chunk(const LinearArgs* const* jobs, int count, int nt, 
     if ((float*)jobs[i]->work < g.partial) g.partial = (float*)jobs[i]->work;
   int64_t wg = 0, cw = 0;
   for (int i = 0; i < count; ++i) {
-    const LinearArgs& a = *jobs[i];
+    const LinearArgs& a = *order[(size_t)i];
     LinearGroupJob& jb = g.job[i];
     jb.x = (const __bf16*)a.x;
     jb.latent = (const __bf16*)a.latent;

@@ -92,3 +92,19 @@ def test_grouped_linear(in_f, out_f, tokens, layers):
     specs = [(x, lat, out_f, layers, 40 + i, 0.5, {"bias": bias} if i % 2 else {}) for i, lat in enumerate(lats)]
     for spec, got in zip(specs, ops.linear_forward_grouped(specs)):
         assert torch.equal(got, ops.linear_forward(*spec[:6], **spec[6]))
+
+
+@pytest.mark.parametrize("in_first", [768, 4096])
+def test_grouped_linear_of_mixed_rows(in_first):
+    """Jobs of short and long rows and of several batches in one launch, whichever comes first:
+    the launch starts the blocks with the most work, each job's outputs are its own call's."""
+    shapes = [(768, 3072, 130), (4096, 700, 5), (3072, 768, 130), (768, 768, 1), (4096, 600, 250)]
+    shapes.sort(key=lambda s: s[0], reverse=in_first == 4096)
+    specs = []
+    for i, (in_f, out_f, tokens) in enumerate(shapes):
+        x = torch.randn(tokens, in_f, generator=torch.Generator().manual_seed(i)).to(BF16).cuda()
+        bias = torch.randn(out_f, generator=torch.Generator().manual_seed(out_f)).to(BF16).cuda()
+        specs.append((x, latent_for(20000 + 7 * i, i).cuda(), out_f, 3, 40 + i, 0.5, {"bias": bias} if i % 2 else {}))
+    assert sum((x.shape[1] * out_f + B - 1) // B for x, _, out_f, *_ in specs) > 256
+    for spec, got in zip(specs, ops.linear_forward_grouped(specs)):
+        assert torch.equal(got, ops.linear_forward(*spec[:6], **spec[6]))
