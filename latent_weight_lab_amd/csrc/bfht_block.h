@@ -434,8 +434,9 @@ struct BwdLds {
   static constexpr int FLOATS = kMost > 256 ? kMost : 256;
 };
 
-template <int LB>
-inline constexpr bool kBwdSingle = LB >= 11 && LB <= 14;  // has a kLoop = false variant
+// Has a kLoop = false variant, for gradients of type Grad.
+template <int LB, class Grad>
+inline constexpr bool kBwdSingle = LB >= 11 && (LB < 15 || sizeof(Grad) == 2);
 
 // Backward of whole blocks: the adjoint chain D_0 H D_1 ... H D_L on grad scattered
 // into each block, summed over a run of blocks.  A workgroup takes the G blocks
@@ -450,9 +451,13 @@ inline constexpr bool kBwdSingle = LB >= 11 && LB <= 14;  // has a kLoop = false
 // latent 2^15, 96 -> 69 us (now bound by the vector unit's butterflies, as the
 // forward is); 2^12, 98 -> 55; 2^10, 231 -> 38; 2^6, 3040 -> 79.  A latent of 1000
 // under 4000 values: one row, so no second launch, 10.2 -> 6.9 us.
-// kLoop = false (one range per workgroup, 2^11 .. 2^14): no sum over ranges, no
-// registers for it (2^14 under 2^22 values took 18.7 us with them, 16.7 without;
-// at 2^15 it made no difference).
+// kLoop = false (one range per workgroup, from 2^11): no sum over ranges, no
+// registers for it (2^14 under 2^22 values took 18.7 us with them, 16.7 without).
+// 2^15: only for 16-bit gradients (float16, two blocks, two layers: 16.5 -> 16.0 us);
+// with float32 ones that variant is the slower (two blocks, three layers: 18.2 with
+// the sum's registers, 19.1 without).  Several ranges: at 128 registers, which two or
+// four workgroups per CU need, the sum spills 18 and 21 at 2^11 and 2^12, up to 10 at
+// other sizes (4096 values, 2592 blocks: 43.1 us with a row per block, 36.9 so).
 template <int LB, class T, bool kLoop, class Load>
 __device__ __forceinline__ void block_bwd_row(Load grad, float* __restrict__ row, T* __restrict__ grad_latent, int n,
                                               int64_t first_block, int64_t index, int run, int64_t start,

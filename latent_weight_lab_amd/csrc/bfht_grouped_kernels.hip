@@ -68,14 +68,14 @@ template <int LB, class T, class W>
 hipError_t launch_lb(const GroupTable& g, hipStream_t s, bool fwd) {
   if (group_slots_per_wg(LB) != Geo<LB>::G) return hipErrorInvalidValue;  // the planner's prefix unit
   const dim3 grid((unsigned)g.prefix[g.count]), block(Geo<LB>::WG);
-  bool loop = !kBwdSingle<LB>;
+  bool loop = !kBwdSingle<LB, W>;
   for (int j = 0; j < g.count; ++j) loop = loop || g.job[j].run > 1;
   if (fwd)
     hipLaunchKernelGGL((bfht_block_fwd_grouped<LB, T, W>), grid, block, 0, s, g);
   else if (loop)
     hipLaunchKernelGGL((bfht_block_bwd_grouped<LB, T, W, true>), grid, block, 0, s, g);
   else
-    hipLaunchKernelGGL((bfht_block_bwd_grouped<LB, T, W, !kBwdSingle<LB>>), grid, block, 0, s, g);
+    hipLaunchKernelGGL((bfht_block_bwd_grouped<LB, T, W, !kBwdSingle<LB, W>>), grid, block, 0, s, g);
   return hipGetLastError();
 }
 

@@ -723,7 +723,7 @@ static hipError_t launch_block_bwd(const BfhtArgs& a, hipStream_t s) {
   const int64_t run = block_bwd_run(LB, a.nblocks), rows = block_bwd_rows(LB, a.nblocks);
   const int direct = rows == 1;
   const auto kernel =
-      kBwdSingle<LB> && run == 1 ? &bfht_block_bwd<LB, T, !kBwdSingle<LB>> : &bfht_block_bwd<LB, T, true>;
+      kBwdSingle<LB, T> && run == 1 ? &bfht_block_bwd<LB, T, !kBwdSingle<LB, T>> : &bfht_block_bwd<LB, T, true>;
   hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(Gm::WG), 0, s, (const T*)a.src, (float*)a.work, (T*)a.dst,
                      (int)a.n, a.first_block, a.start, a.stop, a.seed32, a.layers, (int)run, direct);
   hipError_t e = hipGetLastError();
