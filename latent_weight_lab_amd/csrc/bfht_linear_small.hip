@@ -53,12 +53,15 @@ constexpr int kSpan = 8;  // k iterations of a lane whose x loads are in flight 
 // then (over them, once they are read) the weight tile and the staged x of one
 // token quad, 4096 values of it, so that a 2^14 block takes 80 KiB and two
 // workgroups share a CU.  Wide: the weight tile behind the generator's LDS, which
-// holds a single token's staged x afterwards; one workgroup per CU at 2^14, two below.
+// holds a single token's staged x afterwards; one workgroup per CU at 2^14, two
+// below, and no barrier before the tile's stores.
+constexpr int kQuadStage = 4096;
 template <int LB, bool kWide>
 struct SmallLinearGeo {
   using Gm = Geo<LB>;
   static constexpr int kTileElems = Gm::G * Gm::B;  // weights generated per workgroup
-  static constexpr int kStage = kWide ? BlockLds<LB>::FLOATS : 4096;
+  static constexpr int kStage = kWide ? BlockLds<LB>::FLOATS : kQuadStage;
+  static_assert(!kWide || kStage >= Gm::B, "one token's row fits the generator's LDS");
   static constexpr int kTile = kWide ? BlockLds<LB>::FLOATS : 0;   // where the weight tile starts
   static constexpr int kStaged = kWide ? 0 : kTileElems;           // and the staged x
   static constexpr int kNeed = kTileElems + kStage;
@@ -329,7 +332,10 @@ hipError_t launch_small_lb(const LinearArgs& a, hipStream_t s) {
   using Gm = Geo<LB>;
   const int64_t wtiles = (a.nblocks_w + Gm::G - 1) / Gm::G;
   const int log_in = log2_of(a.in_features);
-  // The narrow form wherever it stages a quad's x.  A longer row is staged alone (one
+  // The narrow form wherever it stages a quad's x, but for a single token under at most one
+  // workgroup per CU, which gain nothing from a second and take the wide form, without the
+  // narrow one's barrier before the stores (float16 1024 -> 4096: 12.2 -> 11.7 us; with more
+  // tokens the narrow form is as fast or faster).  A longer row is staged alone (one
   // token, wide: 16384 -> 1000 in float32 107 -> 65 us) or read by every team from the
   // caches (several tokens): with a quad staged in rounds its loads were waited out
   // between barriers (4096 -> 1000, 1000 tokens: float32 1981 -> 715 us, float16 2034 ->
@@ -345,8 +351,8 @@ hipError_t launch_small_lb(const LinearArgs& a, hipStream_t s) {
   const bool one_per_cu = wtiles * a.token_splits <= device_cus();
   const bool streams_x = sizeof(T) == 4 && a.tokens * a.in_features * 4 >= ((int64_t)48 << 20) &&
                          (double)(a.tokens * a.in_features) * (double)(a.in_features * a.out_features) >= 5e14;
-  const bool wide =
-      LB > 10 && nstage > SmallLinearGeo<LB, false>::kStage && (a.tokens == 1 || one_per_cu || streams_x);
+  const bool wide = LB > 10 && (nstage > kQuadStage ? a.tokens == 1 || one_per_cu || streams_x
+                                                    : a.tokens == 1 && one_per_cu);
 #define LWL_SMALL(W)                                                                                                \
   hipLaunchKernelGGL((bfht_linear_small<LB, T, W>), dim3((unsigned)wtiles, (unsigned)a.token_splits), dim3(Gm::WG), \
                      0, s, (const T*)a.x, (const T*)a.latent, (T*)a.out, (int)a.tokens, (int)a.in_features, log_in, \
@@ -431,7 +437,7 @@ bool linear_small_groupable(const LinearArgs& a) {
   // count and tile count stay far below 2^31 (tokens * out and in * out do)
   return linear_small_applicable(a.dtype, a.log_block, a.in_features) && !linear_small_mm_applicable(a) &&
          a.token_splits == 1 && a.nblocks_w < ((int64_t)1 << 24) &&
-         small_stage(a.tokens, a.in_features) <= SmallLinearGeo<kLinearSmallMaxLog, false>::kStage;
+         small_stage(a.tokens, a.in_features) <= kQuadStage;
 }
 
 hipError_t launch_linear_small_grouped(const LinearArgs* jobs, int64_t count, hipStream_t s) {
