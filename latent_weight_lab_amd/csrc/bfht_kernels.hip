@@ -69,9 +69,8 @@ __global__ __launch_bounds__(Geo<LB>::WG, 4) void bfht_block_bwd(const T* __rest
                               first_block, blockIdx.x, run, start, stop, seed32, layers, smem);
 }
 
-// grad_latent[p] = sum_b part[b * stride + p], blocks in order.
-// Fixed-order sum of the per-block float32 partial rows: grad[p] = sum over b
-// of part[b * stride + p].  Each workgroup owns 128 columns (2 per lane); wave
+// Fixed-order sum of the partial rows (one per workgroup of the backward): grad[p] =
+// sum over b of part[b * stride + p].  Each workgroup owns 128 columns (2 per lane); wave
 // w adds rows w, w + 8, w + 16, ... in ascending order with 16 row loads in
 // flight, and wave 0 adds the 8 wave sums in wave order, so the result does
 // not depend on timing.  (A single column walk per thread keeps only a few
@@ -452,7 +451,7 @@ __device__ __forceinline__ void reg_butterflies(float (&v)[32]) {
 //
 // A pass is bound by the reads and writes of the work buffer beside the vector
 // unit's butterflies, and with one tile at a time a CU does neither during the
-// other's barriers.  So a tile takes half of a CU (66 KiB of LDS, 512 threads,
+// other's barriers.  So a tile takes half of a CU (68 KiB of LDS, 512 threads,
 // 128 registers each) and a second workgroup runs through them.  2^26 float32
 // values of 2^20 blocks, 3 layers: forward 343 us with tiles of 2^15 and one
 // workgroup per CU, 325 with these; backward 345, 328; 2^22 blocks 370, 322 and
@@ -481,6 +480,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void bfht_tile_pass(
   __shared__ float lds[kTilePadded];
   __shared__ uint32_t words[kTileElems / 32];
   static_assert(kTileElems / 32 == kTileThreads, "one sign word per thread");
+  static_assert(2 * (sizeof(lds) + sizeof(words)) <= 160 * 1024, "two workgroups per CU");
   // TL = 0: low tile; TL = LB - 14 (the launcher picks it): high tile of 2^TL rows
   constexpr bool high = TL > 0;
   const int tid = threadIdx.x;

@@ -134,9 +134,9 @@ __host__ __device__ constexpr int linear_lds_steps(int nsteps, int pitch) {
 // chunks (8 per thread) while the other two blocks' chains run.
 constexpr int kStageBytes = 8 * mfma15::kThreads * 16;
 // Table rows: whole 16-row tiles when they fit in the LDS, else the exact row
-// count (the reads of the last row tile then run up to 15 rows past the table,
-// into entries whose output columns are never stored, so an exact table leaves
-// that much LDS free).
+// count (the rows that the last row tile then lacks are read from a row inside
+// the table, and their output columns are never stored).  The slack is no part
+// of the table: it only draws the line of the shapes this kernel takes.
 constexpr int64_t kExactPitchSlack = 16 * 16;
 int linear_pitch(int64_t in_features, int kb, int lds_bytes = kLinearLdsBytes) {
   const int64_t padded = 16 * linear_row_tiles(in_features, kb);
@@ -891,10 +891,11 @@ bool table_fits_shared(int64_t in_features) {
   return linear_table_bytes(in_features, linear_pitch(in_features, 1, kSharedCuLdsBytes)) <= kSharedCuLdsBytes;
 }
 
-// Whether a job's k-major table can be read as `nt` row tiles: the contraction
-// reads rows up to 16 nt - 1 of every k chunk (rows past the job's own are
-// never stored), so the last chunk's reads reach 16 nt - pitch rows past its
-// table; they must stay inside the workgroup's LDS.
+// Which jobs a launch of `nt` row tiles takes: those whose table would fit the
+// LDS with 16 nt rows in its last k chunk.  (Every read stays inside the table,
+// rows past the pitch at a row of it, and columns past the job's own rows are
+// never stored; the line keeps long rows of few row tiles, whose MFMAs on absent
+// rows would be most of their work, out of launches of many.)
 bool table_reads_fit(const LinearArgs& a, int nt) {
   const int64_t pitch = linear_pitch(a.in_features, 1);
   const int64_t steps = linear_steps(a.in_features);
@@ -915,9 +916,10 @@ hipError_t launch_group_chunk(const LinearArgs* const* jobs, int count, int nt, 
     const int64_t tt = (jobs[i]->tokens + kTokTile - 1) / kTokTile;
     min_tiles = tt < min_tiles ? tt : min_tiles;
   }
-  // one pass over every job's blocks fills the chip when there are >= 256 of
-  // them; otherwise split the tokens, as the single-matrix launch does
-  int64_t split = total >= 256 ? 1 : 256 / total;
+  // one pass over every job's blocks fills the chip when there is one per CU;
+  // otherwise split the tokens, as the single-matrix launch does
+  const int64_t cus = device_cus();
+  int64_t split = total >= cus ? 1 : cus / total;
   if (split > min_tiles) split = min_tiles;
   if (split < 1) split = 1;
   share_cu = share_cu && chains_share_cu(total * split);

@@ -69,6 +69,9 @@ struct MmGeo {
   static constexpr int LDS_BYTES = TABLE_BYTES > GEN_BYTES ? TABLE_BYTES : GEN_BYTES;
   static_assert(Gm::LT == LB - 5 && SLOTS * Gm::TB == WG, "32 weights per thread");
   static_assert(LDS_BYTES <= 160 * 1024, "generator and table fit the LDS");
+  // float32 tiles of one 16-row tile: two workgroups per CU (linear_small_mm_token_splits)
+  static constexpr int kPerCu = sizeof(T) == 4 ? 2 : 1;
+  static_assert(kPerCu * LDS_BYTES <= 160 * 1024, "their LDS fits the CU's");
 };
 
 // Table row of W row r in k chunk kc.  A ds_read_b128 serves 16 lanes per LDS
@@ -127,7 +130,8 @@ constexpr int kMmDepth = 4;  // x prefetch distance in k steps
 
 // kMmTok: token tiles (of 16) per item.
 template <int LB, class T, int kMmRows, int kMmTok>
-__global__ __launch_bounds__((MmGeo<LB, T>::WG)) void bfht_linear_small_mm(const T* __restrict__ x,
+__global__ __launch_bounds__((MmGeo<LB, T>::WG), (MmGeo<LB, T>::WG / 256) * (kMmRows == 1 ? MmGeo<LB, T>::kPerCu : 1)) void
+bfht_linear_small_mm(const T* __restrict__ x,
                                                                     const u32x4m* __restrict__ xt,
                                                                     const T* __restrict__ latent,
                                                                     T* __restrict__ out, int tokens, int in_f,
@@ -293,8 +297,11 @@ hipError_t launch_mm_lb(const LinearArgs& a, const u32x4m* xt, hipStream_t s) {
   // row tiles per item: the tile's 16-row tiles (rows of one tile, or all of out), at most 4
   const int64_t rows = std::min<int64_t>(MG::TILE >> log_in, a.out_features);
   const int rt = rows > 32 ? 4 : rows > 16 ? 2 : 1;
-  // four token tiles per item, two where four row tiles would leave 16 waves'
-  // 128 VGPRs too few
+  // four token tiles per item, two with four row tiles.  16 waves have 128 VGPRs each, which is
+  // tight: two row tiles spill 11 (blocks of 2^14) to 26 (2^9), one or four up to 10 at 2^7 ..
+  // 2^9; so do 16-row float32 tiles of 2^7 .. 2^9, held to two workgroups per CU.  Against 8
+  // waves of 249 VGPRs without spills and two generator calls: 1024 -> 4096, block 2^14,
+  // float16 24.6 -> 22.0 us at 16 tokens, 36.4 -> 33.7 at 1000, 77.8 -> 74.4 at 4003.
 #define LWL_MM(RT)                                                                                              \
   hipLaunchKernelGGL((bfht_linear_small_mm<LB, T, RT, RT == 4 && sizeof(T) == 2 ? 2 : 4>), dim3((unsigned)wtiles, (unsigned)a.token_splits),     \
                      dim3(MG::WG), 0, s, (const T*)a.x, xt, (const T*)a.latent, (T*)a.out, (int)a.tokens,      \
@@ -347,14 +354,14 @@ int linear_small_mm_token_splits(const LinearArgs& a) {
   // run at once and no more (a split past that costs a second round: 1024 ->
   // 1000 in float32, 4003 tokens, 315 workgroups one per CU 160 us, 504 two per
   // CU 96), at least 64 tokens per split.  One workgroup per CU; float32 tiles of one
-  // 16-row tile fit two (76 KiB of LDS, 118 VGPRs), whose matrix products then
+  // 16-row tile fit two (74 KiB of LDS, at most 128 VGPRs), whose matrix products then
   // overlap: 1024 -> 4096 at 4003 tokens 313 -> 299 us, about even at 1000, and
   // below that the second generation costs more (300 tokens: 50 against 56).
   const int64_t tile = a.dtype == kF32 ? 16384 : 32768;
   const int64_t wtiles = (a.in_features * a.out_features + tile - 1) / tile;
   const int64_t rows = std::min<int64_t>(tile / a.in_features, a.out_features);
   const int64_t per_cu = a.dtype == kF32 && rows <= 16 && a.tokens >= 1024 ? 2 : 1;
-  int64_t split = per_cu * 256 / wtiles;
+  int64_t split = per_cu * device_cus() / wtiles;
   const int64_t most = (a.tokens + 63) / 64;
   if (split > most) split = most;
   if (split > 65535) split = 65535;

@@ -351,7 +351,9 @@ __device__ __forceinline__ void add_signed(f32x16 (&sum)[kTiles], const f32x16 (
 // one bfloat16 row, so a call of more blocks than CUs leaves about one row per
 // CU for the block sum instead of one per block, and the next block's gradient
 // loads while the current one transforms.  One workgroup per CU: the chain, the
-// sum (64 registers) and the loads in flight (32) take up to 256 VGPRs.  Three
+// sum (64 registers) and the loads in flight (32) take 244 VGPRs with kWhole; the
+// paths for partial blocks and off the 16-byte grid take all 256 and spill 33 (136
+// bytes per lane), which the grouped flush, of whole and partial blocks alike, pays too.  Three
 // layers, block sum included, against a row per block (two workgroups per CU):
 // 257 blocks 17.8 / 16.3 us, 300 18.1 / 18.4, 600 24.6 / 25.1, 1024 32.2 / 35.2,
 // 2592 67 / 88 (of which the sum of 2592 rows takes 32); a gradient off the

@@ -68,7 +68,6 @@ constexpr int kChunks = kB / 8;  // 16-byte chunks of 8 bf16 in one block
 // bytes apart, so one ds_read2_b64 fetches a whole MFMA operand into
 // consecutive registers; two buffers back to back (128 KiB).
 constexpr int kXBufBytes = kChunks * 16;
-constexpr int kLdsBytes = 2 * kXBufBytes;
 // Sign-word table after the exchange buffers: the words of sign layers 1..L
 // (1024 per layer, 32 positions each), hashed once per block while the
 // block's source loads are in flight.  A chain kernel's LDS is

@@ -1,5 +1,5 @@
 // lwl_bfht_backward_noalloc: the latent-gradient backward of lwl_bfht_backward
-// with its scratch (one partial row per overlapped block, or the float32 work
+// with its scratch (room for one partial row per overlapped block, or the float32 work
 // buffer of the multi-pass blocks) taken from a file-scope device array instead
 // of a caller-provided workspace, for callers that cannot allocate (code under
 // HIP graph capture, tight serving loops).
