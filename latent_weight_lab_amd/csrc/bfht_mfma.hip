@@ -351,13 +351,16 @@ __device__ __forceinline__ void add_signed(f32x16 (&sum)[kTiles], const f32x16 (
 // one bfloat16 row, so a call of more blocks than CUs leaves about one row per
 // CU for the block sum instead of one per block, and the next block's gradient
 // loads while the current one transforms.  One workgroup per CU: the chain, the
-// sum (64 registers) and the loads in flight (32) take 244 VGPRs with kWhole; the
-// paths for partial blocks and off the 16-byte grid take all 256 and spill 33 (136
-// bytes per lane), which the grouped flush, of whole and partial blocks alike, pays too.  Three
+// sum (64 registers) and the loads in flight (32) take up to 256 VGPRs.  The offsets
+// of the loads of partial blocks, and of blocks off the 16-byte grid at each of its
+// shifts, are the same for every block: the lane is hidden from the compiler before
+// them, which would keep them all over the loop and spill 33 registers for it.  Three
 // layers, block sum included, against a row per block (two workgroups per CU):
 // 257 blocks 17.8 / 16.3 us, 300 18.1 / 18.4, 600 24.6 / 25.1, 1024 32.2 / 35.2,
 // 2592 67 / 88 (of which the sum of 2592 rows takes 32); a gradient off the
-// 16-byte grid, read without prefetch, 128 / 134 at 2564 blocks.
+// 16-byte grid, read without prefetch, 21.8 at 257 blocks, 29.0 at 513 and 91 at 2592
+// (with the offsets kept 28.3, 37.2 and 127; a row per block and one workgroup per CU
+// 24.3, 33.9 and 136).
 template <int L, bool kWhole>
 __device__ __forceinline__ void bwd_sum_row(const __bf16* __restrict__ grad, __bf16* __restrict__ row,
                                             int64_t stride, int64_t first_block, int64_t b0, int64_t b1,
@@ -380,7 +383,9 @@ __device__ __forceinline__ void bwd_sum_row(const __bf16* __restrict__ grad, __b
     } else {
       const int lo = kWhole ? 0 : (int)(start - base > 0 ? start - base : 0);
       const int hi = kWhole ? kB : (int)(stop - base < kB ? stop - base : kB);
-      load_grad<kWhole>(x, gblk, grad + (stop - start), lo, hi, src);
+      Ctx xl = x;
+      if constexpr (!kWhole) asm volatile("" : "+v"(xl.lane32));  // see above
+      load_grad<kWhole>(xl, gblk, grad + (stop - start), lo, hi, src);
     }
     // only the last block of a call can be partial after its first
     loaded = b + 1 < b1 && (kWhole || grad_whole(gblk + kB, 0, (int)(stop - base - kB < kB ? stop - base - kB : kB)));
