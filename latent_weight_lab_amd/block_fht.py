@@ -551,7 +551,7 @@ def prepare_block_fht_weight_cache(model: nn.Module, dtype: torch.dtype | None =
     # jobs are chosen by block size and dtypes, so that only what the kernels take is
     # allocated and packed, the library checks all of them in the one call, and plain
     # weights are made in their final shape (24 float32 latents, bfloat16 weights, prepare
-    # and flush together: 515 us with a library check and views per module, 350 so).
+    # and flush together: 528 us with a library check and views per module, 365 so).
     grouped, specs, shapes = [], [], []
     for module in model.modules():
         if not isinstance(module, BlockFHTLinear) or not _cacheable(module):
