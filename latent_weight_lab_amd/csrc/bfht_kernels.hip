@@ -155,10 +155,12 @@ __device__ __forceinline__ bool reduce_columns(const P* __restrict__ part, int64
         for (int e = 0; e < kVec; ++e) a[e] = ok ? a[e] + lanes(v[j], e) : a[e];
       }
     }
-  } else if (c0 < n) {
-    // the tail of the row: element loads, columns past n read column 0 (a lane with none of
-    // its columns in the row has nothing to add: its loads made the last workgroup wait out
-    // a second round: backward of 255 blocks of 2^12, latent 3000, float32, 16.3 -> 12.9 us)
+  } else if (__builtin_amdgcn_ballot_w64(c0 < n) != 0) {
+    // the tail of the row: element loads, columns past n read column 0.  Lanes with none of
+    // their columns in the row have nothing to add, and without a lane that has some the
+    // wave skips it (backward of 255 blocks of 2^12, latent 3000, float32: 16.3 -> 12.9 us;
+    // a branch per lane instead took the loads of short rows apart: grouped flush of two
+    // latents below 4000 values 26 -> 33 us)
     for (int64_t b0 = wave; b0 < nblocks; b0 += (int64_t)kRedWaves * kRedDepth) {
       float v[kRedDepth][kVec];
 #pragma unroll
