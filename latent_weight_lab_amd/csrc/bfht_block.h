@@ -525,6 +525,13 @@ __device__ __forceinline__ void block_bwd_row(Load grad, float* __restrict__ row
     else
       write(S::lo(0), S::nb(0));
   } else {
+    auto write = [&](int p, float s) {
+      if (p >= n) return;
+      if (grad_latent)
+        grad_latent[p] = from_f32<T>(s);
+      else
+        row[p] = s;
+    };
     float* mine = smem + gi * Gm::PADDED;
     if constexpr (Gm::NG <= 1) {
 #pragma unroll
@@ -542,19 +549,17 @@ __device__ __forceinline__ void block_bwd_row(Load grad, float* __restrict__ row
         put(S::lo(0), S::nb(0));
     }
     __syncthreads();
+    // a call's only block (uniform) has nothing to be added to (a latent of 9 values: 3.1 -> 2.9 us)
+    if (grad_latent != nullptr && stop <= (first_block + 1) * B) {
+      for (int p = threadIdx.x; p < B; p += Gm::WG) write(p, smem[lds_index(p)]);
+      return;
+    }
     // Position p of every thread group: below 256 positions the 256 threads
     // split the groups into chunks, whose sums are added in a second step.
     static_assert(Gm::WG == 256, "several blocks per workgroup of 256 threads");
     constexpr int kCols = B < 256 ? B : 256;
     constexpr int kChunks = 256 / kCols, kPer = G / kChunks;
     const int tid = threadIdx.x, c = tid / kCols;
-    auto write = [&](int p, float s) {
-      if (p >= n) return;
-      if (grad_latent)
-        grad_latent[p] = from_f32<T>(s);
-      else
-        row[p] = s;
-    };
 #pragma unroll 4
     for (int p = tid & (kCols - 1); p < B; p += kCols) {
       float s = 0.0f;
